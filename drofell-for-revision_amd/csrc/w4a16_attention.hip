@@ -335,7 +335,8 @@ paged_attention_reduce_kernel(uint16_t* __restrict__ out, int64_t o_stride, int 
 }
 
 // One workgroup per token: its key and value rows go to their slot.
-// restore: the reverse copy (slots to the token-major tensors).
+// restore: the reverse copy (slots to the token-major tensors).  Used where
+// the token rows are not 16-byte aligned; cache_tile_kernel takes the rest.
 __global__ void reshape_and_cache_kernel(uint16_t* __restrict__ key, int64_t key_stride,
                                          uint16_t* __restrict__ value, int64_t value_stride,
                                          const int64_t* __restrict__ kptr,
@@ -362,6 +363,152 @@ __global__ void reshape_and_cache_kernel(uint16_t* __restrict__ key, int64_t key
       kc[kt] = key[tok * key_stride + i];
       vc[vt] = value[tok * value_stride + i];
     }
+  }
+}
+
+// Token rows to their cache slots (RESTORE: back), one workgroup per (32
+// tokens, kv head).  HBM-bound: every byte is read and written once, so what
+// counts is that both sides move whole 16-byte units in 128-byte runs.
+//   * keys: a 16-byte unit (8 dims of a token) is contiguous on both sides; a
+//     wave takes 8 tokens x 8 units, 128-byte runs of the rows and, for
+//     consecutive slots, of the cache block;
+//   * values: a cache row holds one dim of a block's tokens, so the tile is
+//     turned around in LDS.  Eight tokens in consecutive slots that start at
+//     a multiple of 8 (a "cell") move as one 16-byte unit per dim; the other
+//     tokens (ends of a run, scattered slots, blocks whose address is not
+//     16-byte aligned) as 2-byte elements.  Tiles start slots[0] % 8 tokens
+//     early, so a run that continues a half-filled cell still meets the
+//     tile in whole cells.
+// Measured, 1500 tokens x 32 heads x 128 written and read back: 67.7 -> 25.8 us
+// against element-wise copies (2-byte stores, one workgroup per token).
+constexpr int kCacheTile = 32;                 // tokens per workgroup
+constexpr int kCacheSlab = 128;                // dims per pass
+constexpr int kCachePitch = kCacheSlab + 4;    // halfs per LDS row: the 4 cells of a dim pair
+                                               // read 4 x 16 distinct banks
+
+template <bool RESTORE>
+__global__ void __launch_bounds__(256)
+cache_tile_kernel(uint16_t* __restrict__ key, int64_t key_stride, uint16_t* __restrict__ value,
+                  int64_t value_stride, const int64_t* __restrict__ kptr,
+                  const int64_t* __restrict__ vptr, const int64_t* __restrict__ slots,
+                  int num_tokens, int head_size, int bs_log2, int kv_head_stride) {
+  __shared__ __attribute__((aligned(16))) uint16_t tile[kCacheTile * kCachePitch];
+  __shared__ int64_t slot_s[kCacheTile];
+  __shared__ uint16_t* kbase[kCacheTile];  // token's block (this head), null: skip the token
+  __shared__ uint16_t* vbase[kCacheTile];
+  __shared__ int cell_ok[kCacheTile / 8];
+  const int tid = threadIdx.x;
+  const int head = blockIdx.y;
+  const int bs = 1 << bs_log2;
+  const int64_t first = slots[0];
+  const int t0 = (int)blockIdx.x * kCacheTile - (first >= 0 ? (int)(first & 7) : 0);
+  if (tid < kCacheTile) {
+    const int t = t0 + tid;
+    const int64_t slot = t >= 0 && t < num_tokens ? slots[t] : -1;
+    slot_s[tid] = slot;
+    kbase[tid] = nullptr;
+    vbase[tid] = nullptr;
+    if (slot >= 0) {
+      const int64_t blk = slot >> bs_log2;
+      kbase[tid] = reinterpret_cast<uint16_t*>(kptr[blk]) + (size_t)head * kv_head_stride;
+      vbase[tid] = reinterpret_cast<uint16_t*>(vptr[blk]) + (size_t)head * kv_head_stride;
+    }
+  }
+  __syncthreads();
+  if (tid < kCacheTile / 8) {
+    const int64_t s0 = slot_s[tid * 8];
+    bool ok = s0 >= 0 && (s0 & 7) == 0 &&
+              (reinterpret_cast<uintptr_t>(vbase[tid * 8]) & 15) == 0;
+    for (int i = 1; i < 8; ++i) ok = ok && slot_s[tid * 8 + i] == s0 + i;
+    cell_ok[tid] = ok;
+  }
+  __syncthreads();
+  const int off_mask = bs - 1;
+  const bool singles = !(cell_ok[0] & cell_ok[1] & cell_ok[2] & cell_ok[3]);
+  uint16_t* const krow = key + (size_t)head * head_size;
+  uint16_t* const vrow = value + (size_t)head * head_size;
+
+  for (int d0 = 0; d0 < head_size; d0 += kCacheSlab) {
+    const int nd = min(kCacheSlab, head_size - d0);  // a multiple of 8
+    const int nu = nd / 8;
+    // ---- keys, 16-byte units: 8 tokens x 8 units per wave
+    for (int i = tid; i < kCacheTile * (kCacheSlab / 8); i += 256) {
+      const int w = i >> 6, l = i & 63;
+      const int t = (w & 3) * 8 + (l & 7);
+      const int u = (w >> 2) * 8 + (l >> 3);
+      if (u >= nu || kbase[t] == nullptr) continue;
+      uint16_t* row = krow + (size_t)(t0 + t) * key_stride + d0 + u * 8;
+      uint16_t* unit = kbase[t] + ((size_t)(d0 / 8 + u) * bs + (int)(slot_s[t] & off_mask)) * 8;
+      uint16_t* const dst = RESTORE ? row : unit;
+      const uint16_t* const src = RESTORE ? unit : row;
+      if ((reinterpret_cast<uintptr_t>(unit) & 15) == 0) {
+        *(u4*)dst = *(const u4*)src;
+      } else {
+        for (int e = 0; e < 8; ++e) dst[e] = src[e];
+      }
+    }
+    // ---- values
+    auto rows = [&](auto&& move) {  // (tile address, row address) per 16-byte unit of a token
+      for (int i = tid; i < kCacheTile * (kCacheSlab / 8); i += 256) {
+        const int t = i / (kCacheSlab / 8), u = i % (kCacheSlab / 8);
+        if (u >= nu || vbase[t] == nullptr) continue;
+        move(&tile[t * kCachePitch + u * 8], vrow + (size_t)(t0 + t) * value_stride + d0 + u * 8);
+      }
+    };
+    auto cells = [&](auto&& move) {  // (tile address of the cell's first token, cache address)
+      for (int i = tid; i < (kCacheTile / 8) * (kCacheSlab / 2); i += 256) {
+        const int c = i % (kCacheTile / 8), dp = i / (kCacheTile / 8);
+        if (2 * dp >= nd || !cell_ok[c]) continue;
+        move(&tile[c * 8 * kCachePitch + 2 * dp],
+             vbase[c * 8] + (size_t)(d0 + 2 * dp) * bs + (int)(slot_s[c * 8] & off_mask));
+      }
+    };
+    auto elements = [&](auto&& move) {  // tokens outside whole cells
+      if (!singles) return;
+      for (int i = tid; i < kCacheTile * kCacheSlab; i += 256) {
+        const int t = i % kCacheTile, d = i / kCacheTile;
+        if (d >= nd || cell_ok[t >> 3] || vbase[t] == nullptr) continue;
+        move(&tile[t * kCachePitch + d],
+             vbase[t] + (size_t)(d0 + d) * bs + (int)(slot_s[t] & off_mask));
+      }
+    };
+    if (!RESTORE) {
+      rows([](uint16_t* lds, const uint16_t* row) {
+        const u4 v = *(const u4*)row;
+        *(uint2*)lds = make_uint2(v[0], v[1]);
+        *(uint2*)(lds + 4) = make_uint2(v[2], v[3]);
+      });
+      __syncthreads();
+      cells([&](const uint16_t* lds, uint16_t* dst) {
+        u4 lo, hi;  // 8 tokens of the even and of the odd dim
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const uint32_t a = *(const uint32_t*)(lds + (2 * e) * kCachePitch);
+          const uint32_t b = *(const uint32_t*)(lds + (2 * e + 1) * kCachePitch);
+          lo[e] = (a & 0xFFFFu) | (b << 16);
+          hi[e] = (a >> 16) | (b & 0xFFFF0000u);
+        }
+        *(u4*)dst = lo;
+        *(u4*)(dst + bs) = hi;
+      });
+      elements([](const uint16_t* lds, uint16_t* dst) { *dst = *lds; });
+    } else {
+      cells([&](uint16_t* lds, const uint16_t* src) {
+        const u4 lo = *(const u4*)src, hi = *(const u4*)(src + bs);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          *(uint32_t*)(lds + (2 * e) * kCachePitch) = (lo[e] & 0xFFFFu) | (hi[e] << 16);
+          *(uint32_t*)(lds + (2 * e + 1) * kCachePitch) = (lo[e] >> 16) | (hi[e] & 0xFFFF0000u);
+        }
+      });
+      elements([](uint16_t* lds, const uint16_t* src) { *lds = *src; });
+      __syncthreads();
+      rows([](const uint16_t* lds, uint16_t* row) {
+        const uint2 a = *(const uint2*)lds, b = *(const uint2*)(lds + 4);
+        *(u4*)row = u4{a.x, a.y, b.x, b.y};
+      });
+    }
+    if (d0 + kCacheSlab < head_size) __syncthreads();  // the next slab reuses the tile
   }
 }
 
@@ -576,6 +723,18 @@ hipError_t launch_reshape_and_cache(uint16_t* key, int64_t key_stride, uint16_t*
                                     const int64_t* slots, int num_tokens, int num_kv_heads,
                                     int head_size, int block_size, int kv_head_stride,
                                     bool restore, hipStream_t stream) {
+  // whole 16-byte units on the rows' side (the kernel itself checks the
+  // blocks' addresses); rows that are not take the element-wise copy
+  const bool vec = ((reinterpret_cast<uintptr_t>(key) | reinterpret_cast<uintptr_t>(value)) & 15) == 0 &&
+                   key_stride % 8 == 0 && value_stride % 8 == 0;
+  if (vec) {
+    const dim3 grid((unsigned)((num_tokens + 7 + kCacheTile - 1) / kCacheTile), (unsigned)num_kv_heads);
+    const int bs_log2 = block_size == 16 ? 4 : 5;
+    auto kern = restore ? &cache_tile_kernel<true> : &cache_tile_kernel<false>;
+    kern<<<grid, 256, 0, stream>>>(key, key_stride, value, value_stride, kptr, vptr, slots,
+                                   num_tokens, head_size, bs_log2, kv_head_stride);
+    return hipGetLastError();
+  }
   const int n = num_kv_heads * head_size;
   reshape_and_cache_kernel<<<(unsigned)num_tokens, std::min(1024, n), 0, stream>>>(
       key, key_stride, value, value_stride, kptr, vptr, slots, num_kv_heads, head_size,
