@@ -783,50 +783,94 @@ __global__ void reduce_kernel(const float* __restrict__ part, int splits, int M,
 }
 
 // ---------------------------------------------------------------------------
-// Bit-exact dequantisation to the original row order (one thread per 16-byte
-// lane unit = 32 weights).  BF16 writes the fp16 value converted to bf16
-// (round to nearest even; a NaN stays a NaN with the quiet bit set).
+// Bit-exact dequantisation to the original row order.  BF16 writes the fp16
+// value converted to bf16 (round to nearest even).  HBM-bound (K * N / 2
+// bytes read, 2 * K * N written), so what counts is that the stores are
+// whole lines: a packed chunk holds 16 columns, 32 bytes of an output row.
+// A workgroup therefore takes 8 strips of one 128-row chunk, turns them
+// around in LDS (one row = 256 bytes) and stores 16-byte units, 256 bytes
+// of a row at a time.  Values come from the same identity as the GEMMs' (the
+// exact integer q - z, one IEEE fp16 multiply by the scale: not an fp32
+// product narrowed to fp16, which may be contracted into a mixed-precision
+// FMA with a +0 addend that turns a -0 product into +0).
+// Measured over distinct matrices and outputs, against one thread per 16-byte
+// packed unit with 2-byte stores: 4096^2 15.0 -> 10.7 us, 4096 x 11008 36.8 ->
+// 28.0, 11008 x 4096 69.3 -> 28.6, 5120 x 13824 119.5 -> 44.0 (4.0 TB/s; a
+// 1 GiB copy reaches 5.0).
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ uint16_t bf16_of_h(_Float16 v) {
-  const uint32_t f = __builtin_bit_cast(uint32_t, (float)v);  // exact widening
-  if ((f & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((f >> 16) | 0x40u);
-  return (uint16_t)((f + 0x7fffu + ((f >> 16) & 1u)) >> 16);
-}
+constexpr int kDqStrips = 8;                     // strips per workgroup: 256-byte rows
+constexpr int kDqPitch = kDqStrips * kStripN;    // halfs per LDS row
 
 template <bool BF16>
-__global__ void dequant_kernel(const u4* __restrict__ pq, const uint32_t* __restrict__ pz,
-                               const uint16_t* __restrict__ ps, const int32_t* __restrict__ perm,
-                               uint16_t* __restrict__ w, int64_t ldw, int K, int N, int gs, int G) {
-  const size_t o = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const size_t total = (size_t)K * N / 32;
-  if (o >= total) return;
-  const int lane = (int)(o & 63);
-  const size_t unit = o >> 6;
-  const int KC = K / kChunkK;
-  const int c = (int)(unit % KC);
-  const int s = (int)(unit / KC);
-  const int j = lane & 15;
-  const int n = s * kStripN + j;
-  const u4 q = pq[o];
+__global__ void __launch_bounds__(256)
+dequant_kernel(const u4* __restrict__ pq, const uint32_t* __restrict__ pz,
+               const uint16_t* __restrict__ ps, const int32_t* __restrict__ perm,
+               uint16_t* __restrict__ w, int64_t ldw, int K, int N, int gs, int G, bool vec) {
+  // 16-byte unit v of row r is kept at v ^ f(r), f(r) = 8 (r & 1) + 2 (r / 8 & 3):
+  // the rows one store instruction writes (2 adjacent ones of 4 row groups)
+  // then fall on different banks
+  __shared__ __attribute__((aligned(16))) uint16_t tile[kChunkK * kDqPitch];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int j = lane & 15, kq = lane >> 4;
+  const int KC = K / kChunkK, NS = N / kStripN;
+  const int ng = (NS + kDqStrips - 1) / kDqStrips;
+  const int c = blockIdx.x / ng;
+  const int s0 = (blockIdx.x - c * ng) * kDqStrips;
+  const uint32_t magic = opaque(kMagic);
+  auto f = [](int r) { return ((r & 1) << 3) | (((r >> 3) & 3) << 1); };
 #pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    const int k0 = c * kChunkK + 32 * t + 8 * (lane >> 4);
-    const int g = k0 / gs;
-    const uint32_t zw = pz[((size_t)s * G + g) * 2 + (j >> 3)];
-    const int ze = (int)((zw >> ((j & 7) * 4)) & 15u) + 1;
-    const _Float16 sc = as_h(ps[((size_t)s * G + g) * 16 + j]);
+  for (int si = 0; si < kDqStrips / 4; ++si) {
+    const int ls = wave + 4 * si;
+    const int s = s0 + ls;
+    if (s >= NS) continue;  // wave-uniform
+    const u4 q = __builtin_nontemporal_load(pq + ((size_t)s * KC + c) * 64 + lane);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int slot = (e & 1) ? 4 + (e >> 1) : (e >> 1);
-      const int qv = (int)((q[t] >> (4 * slot)) & 15u);
-      // One IEEE fp16 multiply (round to nearest even) of the scale and the
-      // exact integer |q - z| <= 16.  Not written as an fp32 product
-      // narrowed to fp16: that form may be contracted into a mixed-precision
-      // FMA with a +0 addend, which turns a -0 product into +0.
-      const _Float16 v = sc * (_Float16)(qv - ze);
-      const int k = k0 + e;
-      const int row = perm ? perm[k] : k;
-      w[(size_t)row * ldw + n] = BF16 ? bf16_of_h(v) : h_bits(v);
+    for (int t = 0; t < 4; ++t) {
+      const int g = (c * kChunkK + 32 * t) / gs;  // groups hold whole 32-row steps
+      const uint32_t zw = pz[((size_t)s * G + g) * 2 + (j >> 3)];
+      const _Float16 sc = as_h(ps[((size_t)s * G + g) * 16 + j]);
+      h2 nz1024, nz64;
+      zero_consts(zw, (j & 7) * 4, nz1024, nz64);
+      const h8 v = centered8(q[t], nz1024, nz64, magic) * h8{sc, sc, sc, sc, sc, sc, sc, sc};
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        // rows 2p, 2p + 1 of this column (low, high half-word), and the same
+        // of the neighbouring column: even lanes keep row 2p of both
+        // columns, odd lanes row 2p + 1
+        uint32_t own;
+        if constexpr (BF16) {
+          typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+          own = __builtin_bit_cast(uint32_t, b2{(__bf16)(float)v[2 * p], (__bf16)(float)v[2 * p + 1]});
+        } else {
+          own = __builtin_bit_cast(uint32_t, h2{v[2 * p], v[2 * p + 1]});
+        }
+        const uint32_t nb = (uint32_t)__builtin_amdgcn_mov_dpp((int)own, 0xB1, 0xF, 0xF, true);
+        const uint32_t pair = (j & 1) ? __builtin_amdgcn_perm(own, nb, 0x07060302u)
+                                      : __builtin_amdgcn_perm(nb, own, 0x05040100u);
+        const int r = 32 * t + 8 * kq + 2 * p + (j & 1);
+        const int col = ls * kStripN + (j & ~1);
+        *(uint32_t*)(tile + r * kDqPitch + (((col >> 3) ^ f(r)) << 3) + (col & 7)) = pair;
+      }
+    }
+  }
+  __syncthreads();
+  const int n0 = s0 * kStripN;
+#pragma unroll
+  for (int i = 0; i < kChunkK / 16; ++i) {
+    const int r = 16 * i + (tid >> 4), v = tid & 15;
+    const int n = n0 + v * 8;
+    if (n >= N) continue;
+    const int k = c * kChunkK + r;
+    uint16_t* dst = w + (size_t)(perm ? perm[k] : k) * ldw + n;
+    const u4 d = *(const u4*)(tile + r * kDqPitch + ((v ^ f(r)) << 3));
+    if (vec) {
+      *(u4*)dst = d;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        dst[2 * e] = (uint16_t)(d[e] & 0xFFFFu);
+        dst[2 * e + 1] = (uint16_t)(d[e] >> 16);
+      }
     }
   }
 }
@@ -986,22 +1030,28 @@ hipError_t launch_reduce_planes(const float* part, int splits, int M, int N, con
   return hipGetLastError();
 }
 
+template <bool BF16>
+static hipError_t launch_dequant_t(const uint32_t* pq, const uint32_t* pz, const uint16_t* ps,
+                                   const int32_t* perm, uint16_t* w, int64_t ldw, int K, int N,
+                                   int gs, int G, hipStream_t stream) {
+  const int strips = N / kStripN;
+  const unsigned grid = (unsigned)((strips + kDqStrips - 1) / kDqStrips * (K / kChunkK));
+  const bool vec = (reinterpret_cast<uintptr_t>(w) & 15) == 0 && ldw % 8 == 0;
+  dequant_kernel<BF16><<<grid, 256, 0, stream>>>((const u4*)pq, pz, ps, perm, w, ldw, K, N, gs, G,
+                                                 vec);
+  return hipGetLastError();
+}
+
 hipError_t launch_dequant(const uint32_t* pq, const uint32_t* pz, const uint16_t* ps,
                           const int32_t* perm, uint16_t* w, int64_t ldw, int K, int N, int gs, int G,
                           hipStream_t stream) {
-  const size_t total = (size_t)K * N / 32;
-  dequant_kernel<false><<<(unsigned)((total + 255) / 256), 256, 0, stream>>>(
-      (const u4*)pq, pz, ps, perm, w, ldw, K, N, gs, G);
-  return hipGetLastError();
+  return launch_dequant_t<false>(pq, pz, ps, perm, w, ldw, K, N, gs, G, stream);
 }
 
 hipError_t launch_dequant_bf16(const uint32_t* pq, const uint32_t* pz, const uint16_t* ps,
                                const int32_t* perm, uint16_t* w, int64_t ldw, int K, int N, int gs,
                                int G, hipStream_t stream) {
-  const size_t total = (size_t)K * N / 32;
-  dequant_kernel<true><<<(unsigned)((total + 255) / 256), 256, 0, stream>>>(
-      (const u4*)pq, pz, ps, perm, w, ldw, K, N, gs, G);
-  return hipGetLastError();
+  return launch_dequant_t<true>(pq, pz, ps, perm, w, ldw, K, N, gs, G, stream);
 }
 
 // ---------------------------------------------------------------------------
