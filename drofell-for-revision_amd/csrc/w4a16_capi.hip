@@ -68,8 +68,10 @@ int status_of(hipError_t e) { return e == hipSuccess ? DW4_OK : DW4_ERR_LAUNCH; 
 
 size_t prefill_ws_bytes(const dw4::PrefillPlan& p, int m, int n);
 
-// Prefill tiling and split-K factor for one call.  `ws_bytes` caps the
-// split count: with too little workspace the call runs unsplit.
+// Tiling and split-K factor of the register-fed prefill kernels
+// (launch_prefill): act-order calls whose workspace cannot hold the gathered
+// rows, x rows too far apart for 32-bit offsets, and M <= 32.  `ws_bytes`
+// caps the split count: with too little workspace the call runs unsplit.
 dw4::PrefillPlan plan_prefill(int m, int k, int n, int split_req, size_t ws_bytes, bool cap_by_ws) {
   dw4::PrefillPlan p;
   // Row tile: 16 or 32 rows just covering small M, then 64 (above 128 rows
@@ -165,6 +167,115 @@ dw4::PrefillPlan plan_prefill(int m, int k, int n, int split_req, size_t ws_byte
   return p;
 }
 
+// ---------------------------------------------------------------------------
+// Plan of the LDS-streamed (w4a16_prefill.hip) and K-sliced (w4a16_kslice.hip)
+// kernels: the tile shape and K split of least modelled time.
+//
+// A launch runs its workgroups in rounds of `per` per CU.  A round costs a
+// fixed part (ring prologue, cross-wave sums, stores) and a part per 128-row
+// chunk (K-sliced: per chunk of a wave, an eighth of the split's); the chunks
+// of the last round run faster the fewer CUs it fills (clocks, L2).  A K split
+// adds the reduce launch and its fp32 planes (us per MB).  The constants (us)
+// are least-squares fits to 3024 graph-replayed launches: seven 7B and 13B
+// shapes, M = 24..3500, splits 1..8, 256 CUs; mean error 2-4 % per tile, and
+// on the 126 (shape, M > 64) points the pick is 0.1 % slower than the fastest
+// launch measured.  Against the rules this replaces (fewest rounds, fixed
+// preferences by M) the picks are 1.13x faster in the geometric mean:
+// 4096^2 M=256 21.1 -> 16.4 us, 5120^2 M=96 19.9 -> 13.2, 4096 x 11008 M=384
+// 59.0 -> 49.0, 11008 x 4096 M=640 99.0 -> 71.3, 13824 x 5120 M=1500 361 -> 245.
+// ---------------------------------------------------------------------------
+struct StreamTile {
+  int bm, bn, waves, per;
+  bool kslice;
+  float base, round, chunk;      // launch; a full round: fixed, per chunk
+  float round1, chunk1, fill1;   // last round, at most one workgroup per CU: fixed, per chunk,
+                                 // per chunk and fraction of the CUs filled
+  float chunk2, fill2;           // last round of more (per == 2): per chunk, per chunk and
+                                 // fraction of the CUs with two
+  float split, plane;            // K split: launch, per MB of planes
+};
+constexpr StreamTile kStreamTiles[] = {
+    {32, 64, 8, 2, true, 4.71f, 1.46f, 3.53f, 0.39f, 1.16f, 0.66f, 2.80f, 0.61f, 2.07f, 0.374f},
+    {64, 32, 8, 1, true, 2.61f, 2.51f, 1.88f, 1.52f, 1.33f, 0.52f, 0.f, 0.f, 0.69f, 0.787f},
+    {64, 64, 8, 1, true, 4.12f, 2.74f, 2.89f, 2.68f, 1.47f, 1.14f, 0.f, 0.f, 1.23f, 0.299f},
+    {32, 128, 4, 2, false, 5.13f, 1.03f, 0.905f, 0.f, 0.521f, 0.06f, 0.823f, 0.07f, 2.97f, 0.363f},
+    {64, 128, 4, 2, false, 5.64f, 2.17f, 1.234f, 0.59f, 0.572f, 0.12f, 0.944f, 0.23f, 3.26f, 0.324f},
+    {64, 256, 8, 1, false, 5.06f, 3.88f, 1.159f, 2.56f, 0.800f, 0.29f, 0.f, 0.f, 3.09f, 0.222f},
+    {96, 256, 8, 1, false, 5.69f, 4.74f, 1.504f, 3.23f, 0.993f, 0.42f, 0.f, 0.f, 2.84f, 0.220f},
+    {128, 128, 8, 1, false, 3.73f, 7.10f, 1.124f, 5.59f, 0.876f, 0.28f, 0.f, 0.f, 3.51f, 0.265f},
+    {128, 256, 8, 1, false, 5.34f, 5.40f, 1.914f, 4.71f, 1.257f, 0.51f, 0.f, 0.f, 3.18f, 0.213f},
+};
+constexpr int kStreamMaxSplits = 8;
+constexpr int kStreamMinChunks = 4;  // of a split: fewer never paid
+
+size_t stream_ws_bytes(int splits, int m, int n) {
+  return dw4::split_ws_bytes(splits, (size_t)m * n);
+}
+
+// `count` matrices of k x n share x and run as one launch (unsplit for more
+// than one).  split_req > 0 fixes the split count; splits whose planes
+// exceed ws_bytes are left out.  *cost: the modelled time.
+dw4::PrefillPlan plan_stream(int m, int k, int n, int count, int split_req, size_t ws_bytes,
+                             double* cost = nullptr) {
+  const int kc = k / kChunkK;
+  const int cus = cu_count();
+  const int m32 = (m + 31) / 32 * 32;  // one plan for the Ms of equal tile counts
+  dw4::PrefillPlan best;
+  double best_cost = 1e30;
+  const int lo = split_req > 0 ? std::min(split_req, kc) : 1;
+  const int hi = split_req > 0 ? lo : count > 1 ? 1 : kStreamMaxSplits;
+  for (const StreamTile& t : kStreamTiles) {
+    const int64_t tiles =
+        (int64_t)((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn) * count;
+    for (int s = lo; s <= hi; ++s) {
+      const int cps = (kc + s - 1) / s;
+      const int splits = (kc + cps - 1) / cps;
+      if (split_req <= 0 && s > 1 && (cps < kStreamMinChunks || splits != s)) break;
+      // the caller's planes do not fit: that call runs unsplit
+      const bool fits = splits == 1 || stream_ws_bytes(splits, m32, n) <= ws_bytes;
+      if (!fits && split_req <= 0) break;
+      const int real = fits ? splits : 1;
+      const int chunks = real == splits ? cps : kc;
+      const int64_t wgs = tiles * real;
+      const int64_t slots = (int64_t)cus * t.per;
+      const int64_t full = wgs / slots, rem = wgs - full * slots;
+      const double c = t.kslice ? (chunks + 7) / 8 : chunks;
+      const double fill = (double)rem / cus;
+      double us = t.base + (double)full * (t.round + t.chunk * c);
+      if (rem > cus) us += t.round + (t.chunk2 + t.fill2 * (fill - 1.0)) * c;
+      else if (rem > 0) us += t.round1 + (t.chunk1 + t.fill1 * fill) * c;
+      if (real > 1) us += t.split + t.plane * ((double)real * m32 * n * 4e-6);
+      if (us < best_cost) {
+        best_cost = us;
+        best.bm = t.bm;
+        best.bn = t.bn;
+        best.waves = t.waves;
+        best.kslice = t.kslice;
+        best.splits = real;
+      }
+    }
+  }
+  if (cost != nullptr) *cost = best_cost;
+  return best;
+}
+
+// Calls of the streamed kernels: x in the packed row order, rows within
+// 32-bit offsets, more rows than the decode kernels' small tiles.
+constexpr int kStreamMinM = 33;
+// Act-order calls up to this many rows keep the register-fed kernels with or
+// without room for the gathered rows, so that both give the same bits.
+constexpr int kStreamMinMAct = 65;
+
+bool use_stream(int m, int64_t ldx, bool act) {
+  return m >= (act ? kStreamMinMAct : kStreamMinM) && dw4::prefill_x_fits(ldx);
+}
+
+hipError_t launch_stream(const dw4::GroupArgs& g, const dw4::PrefillPlan& plan, void* ws,
+                         hipStream_t stream) {
+  return plan.kslice ? dw4::launch_kslice_group(g, plan, ws, stream)
+                     : dw4::launch_prefill2_group(g, plan, ws, stream);
+}
+
 size_t prefill_ws_bytes(const dw4::PrefillPlan& p, int m, int n) {
   const size_t mt = (size_t)(m + p.bm - 1) / p.bm, nt = (size_t)(n + p.bn - 1) / p.bn;
   return dw4::split_ws_bytes(p.splits, mt * nt * p.bm * p.bn);
@@ -193,8 +304,11 @@ size_t workspace_for(int path, int m, int k, int n, int group_size, bool act) {
     const dw4::DecodePlan p = dw4::plan_decode(m, k, n, group_size, cu_count());
     split = dw4::split_ws_bytes(p.splits, (size_t)m * n);
   } else {
-    const dw4::PrefillPlan p = plan_prefill(m, k, n, 0, 0, false);
-    split = prefill_ws_bytes(p, m, n);
+    // a call takes the streamed or the register-fed kernels by its strides
+    // and room: the size serves either
+    split = prefill_ws_bytes(plan_prefill(m, k, n, 0, 0, false), m, n);
+    if (use_stream(m, 0, act))
+      split = std::max(split, stream_ws_bytes(plan_stream(m, k, n, 1, 0, SIZE_MAX).splits, m, n));
   }
   if (!act) return split;
   return dw4::gather_offset(split) + dw4::gather_bytes(m, k);
@@ -236,7 +350,10 @@ int dw4_query_sizes(int k, int n, int group_size, int act_order, int max_m,
     size_t ws = 0;
     // enough for either explicit path at every M up to max_m
     for (int m = 1; m <= max_m; ++m) {
-      ws = std::max(ws, workspace_for(DW4_PATH_PREFILL, m, k, n, group_size, act_order != 0));
+      // above 128 rows every plan depends on M in steps of 32 rows and grows
+      // within a step
+      if (m <= 128 || m % 32 == 0 || m == max_m)
+        ws = std::max(ws, workspace_for(DW4_PATH_PREFILL, m, k, n, group_size, act_order != 0));
       if (m <= dw4::kDecodeMaxM)
         ws = std::max(ws, workspace_for(DW4_PATH_DECODE, m, k, n, group_size, act_order != 0));
     }
@@ -379,15 +496,28 @@ int gemm_run(int path, int split_k, int m, int k, int n, int group_size, const u
     return status_of(dw4::launch_decode(a, plan, part, s));
   }
 
+  // The streamed kernels, where x is (or can be gathered) in the packed row
+  // order; otherwise the register-fed ones, which gather per workgroup.
+  const size_t room = workspace && aligned16(workspace) ? workspace_bytes : 0;
+  if (use_stream(m, ldx, perm != nullptr)) {
+    dw4::PrefillPlan plan;
+    // act-order: the gathered rows come first; a split only with what is
+    // left (whole 256 bytes, as gather_offset aligns the rows after it)
+    const size_t need = perm != nullptr ? dw4::gather_bytes(m, k) : 0;
+    plan = plan_stream(m, k, n, 1, split_k, room > need ? (room - need) & ~(size_t)255 : 0);
+    const int e = gather_after(plan.splits > 1 ? stream_ws_bytes(plan.splits, m, n) : 0);
+    if (e != DW4_OK) return e;
+    if (a.perm == nullptr) {
+      dw4::GroupArgs g{};
+      g.count = 1;
+      g.a[0] = a;
+      return status_of(launch_stream(g, plan, workspace, s));
+    }
+  }
   dw4::PrefillPlan plan = plan_prefill(m, k, n, split_k, workspace ? workspace_bytes : 0, true);
   if (plan.splits > 1 && !aligned16(workspace)) plan.splits = 1;
   const int e = gather_after(plan.splits > 1 ? prefill_ws_bytes(plan, m, n) : 0);
   if (e != DW4_OK) return e;
-  // above 128 rows the LDS-streamed kernel, which needs x in the packed row
-  // order (act-order calls whose workspace could not hold the gathered rows
-  // keep the kernel that gathers per workgroup)
-  if (m > 128 && a.perm == nullptr)
-    return status_of(dw4::launch_prefill2(a, plan, workspace, s));
   return status_of(dw4::launch_prefill(a, plan, workspace, s));
 }
 
@@ -830,19 +960,23 @@ int dw4_gemm_group(int count, const dw4_item* items, int m, const uint16_t* x, i
       return status_of(dw4::launch_decode_group(g, plan, static_cast<hipStream_t>(stream)));
     }
   }
-  // above 128 rows, matrices of equal N without act-order: one launch of the
-  // LDS-streamed prefill kernel, planned as one matrix of the summed N
-  // (so the tiles fill the CUs as a merged matrix's would), when that plan
-  // needs no K split
-  bool same_n = items[0].perm == nullptr;
-  for (int i = 1; i < count; ++i) same_n = same_n && items[i].n == items[0].n;
-  if (m > 128 && same_n && count > 1) {
-    const dw4::PrefillPlan plan = plan_prefill(m, items[0].k, n_total, 0, 0, false);
-    if (plan.splits == 1) {
+  // Where the matrices would run on the streamed kernels one by one, have
+  // equal N and no act-order permutation: one launch over the column tiles of
+  // all of them, unless the model prefers them one after another (each with
+  // its own K split).
+  bool same = items[0].perm == nullptr && count > 1;
+  for (int i = 1; i < count; ++i) same = same && items[i].n == items[0].n;
+  if (same && use_stream(m, ldx, false) && !use_decode(DW4_PATH_AUTO, m, items[0].k, items[0].n)) {
+    const size_t room = workspace && aligned16(workspace) ? workspace_bytes : 0;
+    double together = 0.0, alone = 0.0;
+    const dw4::PrefillPlan plan =
+        plan_stream(m, items[0].k, items[0].n, count, 0, room, &together);
+    plan_stream(m, items[0].k, items[0].n, 1, 0, room, &alone);
+    if (together <= count * alone) {
       dw4::GroupArgs g{};
       g.count = count;
       for (int i = 0; i < count; ++i) g.a[i] = args_of(m, x, ldx, &items[i]);
-      return status_of(dw4::launch_prefill2_group(g, plan, workspace, static_cast<hipStream_t>(stream)));
+      return status_of(launch_stream(g, plan, workspace, static_cast<hipStream_t>(stream)));
     }
   }
   for (int i = 0; i < count; ++i) {
@@ -877,8 +1011,13 @@ int dw4_gemm_silu_mul(int m, const uint16_t* x, int64_t ldx, const dw4_item* gat
   st = check_output(gate);
   if (st == DW4_OK) st = check_output(up);
   if (st != DW4_OK) return st;
-  st = gemm_item(m, x, ldx, gate, workspace, workspace_bytes, stream);
-  if (st == DW4_OK) st = gemm_item(m, x, ldx, up, workspace, workspace_bytes, stream);
+  if (gate->perm == nullptr) {
+    const dw4_item both[2] = {*gate, *up};
+    st = dw4_gemm_group(2, both, m, x, ldx, workspace, workspace_bytes, stream);
+  } else {  // each gathers x into its own row order
+    st = gemm_item(m, x, ldx, gate, workspace, workspace_bytes, stream);
+    if (st == DW4_OK) st = gemm_item(m, x, ldx, up, workspace, workspace_bytes, stream);
+  }
   if (st != DW4_OK) return st;
   return status_of(dw4::launch_silu_mul(gate->y, gate->ldy, up->y, up->ldy, h, ldh, m, gate->n, s));
 }
@@ -1034,7 +1173,14 @@ extern "C" int dw4_gemm_noalloc(int m, int k, int n, int group_size, const uint1
   if (st != DW4_OK) return st;
   if (m < 0) return DW4_ERR_INVALID_ARG;
   if (m == 0) return DW4_OK;
-  const size_t need = workspace_for(DW4_PATH_AUTO, m, k, n, group_size, perm != nullptr);
+  size_t need = workspace_for(DW4_PATH_AUTO, m, k, n, group_size, perm != nullptr);
+  // a streamed K split is optional: without room for its planes the call
+  // runs unsplit
+  if (need > DW4_NOALLOC_SCRATCH_BYTES && !use_decode(DW4_PATH_AUTO, m, k, n) &&
+      use_stream(m, ldx, perm != nullptr)) {
+    need = prefill_ws_bytes(plan_prefill(m, k, n, 0, 0, false), m, n);
+    if (perm != nullptr) need = dw4::gather_offset(need) + dw4::gather_bytes(m, k);
+  }
   if (need > DW4_NOALLOC_SCRATCH_BYTES) return DW4_ERR_SCRATCH;
   int status = DW4_OK;
   void* ws = scratch_for_current_device(static_cast<hipStream_t>(stream), &status);

@@ -118,10 +118,83 @@ __device__ __forceinline__ float bf16_f32(uint16_t b) {
   return __builtin_bit_cast(float, (uint32_t)b << 16);
 }
 
+// Eight fp32 values rounded to bf16 (v_cvt_pk_bf16_f32, round to nearest even).
+typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
+  return __builtin_bit_cast(uint32_t, b2{(__bf16)lo, (__bf16)hi});
+}
+
+// A column's group constants for the B operands of the prefill kernels.
+// fp16: the weight is fp16(s (q - z)) from the exact integer q - z.
+// bf16: the weight is bf16(s (q - z)), rounded once: with the nibbles OR-ed
+// into fp16 1024.0 (values 1024 + q and 1024 + 16 q), s (1024 + q) - s (1024 +
+// z) is one mixed-precision FMA whose product, addend and result are exact in
+// fp32 (s has 11 significant bits, 1024 + q at most 11, s (q - z) at most 16).
+template <bool BF>
+struct ColGroup;
+template <>
+struct ColGroup<false> {
+  h2 nz1024, nz64;
+  _Float16 s;
+  __device__ __forceinline__ void set(uint32_t sword, int hsh, uint32_t zword, int zsh) {
+    zero_consts(zword, zsh, nz1024, nz64);
+    s = as_h((uint16_t)(sword >> hsh));
+  }
+};
+template <>
+struct ColGroup<true> {
+  float s, c1024, s16, c64;
+  __device__ __forceinline__ void set(uint32_t sword, int hsh, uint32_t zword, int zsh) {
+    s = (float)as_h((uint16_t)(sword >> hsh));
+    const float z = (float)(((zword >> zsh) & 15u) + 1u);
+    c1024 = -s * (1024.f + z);
+    s16 = s * 0.0625f;
+    c64 = -s * (64.f + z);
+  }
+};
+
+// The B operand of 8 rows of one packed word.
+__device__ __forceinline__ h8 weight8(uint32_t w, const ColGroup<false>& g, uint32_t magic) {
+  return centered8(w, g.nz1024, g.nz64, magic) * h8{g.s, g.s, g.s, g.s, g.s, g.s, g.s, g.s};
+}
+__device__ __forceinline__ h8 weight8(uint32_t w, const ColGroup<true>& g, uint32_t magic) {
+  const uint32_t w8 = w >> 8;
+  const h2 p0 = as_h2(and_or(w, 0x000F000Fu, magic)), p1 = as_h2(and_or(w, 0x00F000F0u, magic));
+  const h2 p2 = as_h2(and_or(w8, 0x000F000Fu, magic)), p3 = as_h2(and_or(w8, 0x00F000F0u, magic));
+  return __builtin_bit_cast(
+      h8, u4{pack_bf16(fmaf((float)p0[0], g.s, g.c1024), fmaf((float)p0[1], g.s, g.c1024)),
+             pack_bf16(fmaf((float)p1[0], g.s16, g.c64), fmaf((float)p1[1], g.s16, g.c64)),
+             pack_bf16(fmaf((float)p2[0], g.s, g.c1024), fmaf((float)p2[1], g.s, g.c1024)),
+             pack_bf16(fmaf((float)p3[0], g.s16, g.c64), fmaf((float)p3[1], g.s16, g.c64))});
+}
+
 typedef float f16v __attribute__((ext_vector_type(16)));
 
 __device__ __forceinline__ f16v mfma32(h8 a, h8 b, f16v c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+}
+
+template <bool BF>
+__device__ __forceinline__ f16v mfma32_of(h8 a, h8 b, f16v c) {
+  if constexpr (BF)
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(b8, a),
+                                                   __builtin_bit_cast(b8, b), c, 0, 0, 0);
+  else
+    return mfma32(a, b, c);
+}
+
+// A product rounded to the output type, plus the bias in that type (rounded
+// again, as a tensor add after the product is).
+template <bool BF>
+__device__ __forceinline__ uint16_t round_out(float v, bool has_bias, uint16_t bias) {
+  if constexpr (BF) {
+    const uint16_t o = (uint16_t)pack_bf16(v, 0.f);
+    return has_bias ? (uint16_t)pack_bf16(bf16_f32(o) + bf16_f32(bias), 0.f) : o;
+  } else {
+    _Float16 o = (_Float16)v;
+    if (has_bias) o = o + as_h(bias);
+    return h_bits(o);
+  }
 }
 
 // Two 16-column strips' packed word w (lanes L: column L%16, rows 8(L/16)..)
@@ -175,6 +248,18 @@ __device__ __forceinline__ u4 add_h8(u4 a, u4 b) {
 #pragma unroll
   for (int e = 0; e < 4; ++e) r[e] = __builtin_bit_cast(uint32_t, as_h2(a[e]) + as_h2(b[e]));
   return r;
+}
+
+// Buffer resource over [p, p + 4 GiB): a uniform base, so that loads take a
+// uniform byte offset and a 32-bit lane offset and need no 64-bit address
+// arithmetic on the vector ALU.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_of(const void* p) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, 0xFFFFFFFFu, 0x00027000);
+}
+
+// floor(n / d) for the host's magic = ceil(2^32 / d), or n for magic 0 (d = 1).
+__device__ __forceinline__ int div_by_magic(int n, uint32_t magic) {
+  return magic == 0 ? n : (int)__umulhi((uint32_t)n, magic);
 }
 
 __device__ __forceinline__ float silu_f32(float v) { return v / (1.0f + __expf(-v)); }

@@ -749,6 +749,7 @@ prefill32_kernel(const _Float16* __restrict__ x, int64_t ldx, int M,
   if (tid == 0) __hip_atomic_store(&counters[tile_id], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+template <bool BF>
 __global__ void reduce_kernel(const float* __restrict__ part, int splits, int M, int N,
                               const uint16_t* __restrict__ bias,
                               uint16_t* __restrict__ y, int64_t ldy,
@@ -769,14 +770,13 @@ __global__ void reduce_kernel(const float* __restrict__ part, int splits, int M,
   u4 packed;
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
-    _Float16 out = (_Float16)(e < 4 ? s0[e] : s1[e - 4]);
-    if (bias != nullptr) out = out + as_h(bias[n + e]);
-    if (rsrc != nullptr) out = out + as_h(rsrc[e]);
+    uint32_t h = round_out<BF>(e < 4 ? s0[e] : s1[e - 4], bias != nullptr,
+                               bias != nullptr ? bias[n + e] : 0);
+    if (rsrc != nullptr) h = h_bits(as_h((uint16_t)h) + as_h(rsrc[e]));  // fp16 only
     if (vec) {
-      const uint32_t h = h_bits(out);
       packed[e / 2] = (e & 1) ? (packed[e / 2] | (h << 16)) : h;
     } else {
-      dst[e] = h_bits(out);
+      dst[e] = (uint16_t)h;
     }
   }
   if (vec) *(u4*)dst = packed;
@@ -839,8 +839,7 @@ dequant_kernel(const u4* __restrict__ pq, const uint32_t* __restrict__ pz,
         // columns, odd lanes row 2p + 1
         uint32_t own;
         if constexpr (BF16) {
-          typedef __bf16 b2 __attribute__((ext_vector_type(2)));
-          own = __builtin_bit_cast(uint32_t, b2{(__bf16)(float)v[2 * p], (__bf16)(float)v[2 * p + 1]});
+          own = pack_bf16((float)v[2 * p], (float)v[2 * p + 1]);
         } else {
           own = __builtin_bit_cast(uint32_t, h2{v[2 * p], v[2 * p + 1]});
         }
@@ -1022,11 +1021,13 @@ hipError_t launch_prefill(const GemmArgs& a, const PrefillPlan& plan, void* part
 
 hipError_t launch_reduce_planes(const float* part, int splits, int M, int N, const uint16_t* bias,
                                 uint16_t* y, int64_t ldy, const uint16_t* res, int64_t ldres,
-                                hipStream_t stream) {
+                                hipStream_t stream, bool bf16) {
   const size_t units = (size_t)M * N / 8;
   const bool vec = ((reinterpret_cast<uintptr_t>(y) & 15) == 0) && (ldy % 8 == 0);
-  reduce_kernel<<<(unsigned)((units + 255) / 256), 256, 0, stream>>>(part, splits, M, N, bias, y,
-                                                                     ldy, res, ldres, vec);
+  if (bf16 && res != nullptr) return hipErrorInvalidValue;
+  auto kern = bf16 ? &reduce_kernel<true> : &reduce_kernel<false>;
+  kern<<<(unsigned)((units + 255) / 256), 256, 0, stream>>>(part, splits, M, N, bias, y, ldy, res,
+                                                            ldres, vec);
   return hipGetLastError();
 }
 

@@ -1,6 +1,7 @@
-// gfx950 W4A16 prefill kernel: 64 x 256, 128 x 128 or 128 x 256 output
-// tiles (8 waves), or 32 x 128 and 64 x 128 tiles (4 waves, two workgroups
-// per CU) on v_mfma_f32_32x32x16_f16, activations streamed straight into LDS.
+// gfx950 W4A16 prefill kernel: 64, 96 or 128 x 256 or 128 x 128 output tiles
+// (8 waves), or 32 x 128 and 64 x 128 tiles (4 waves, two workgroups per CU)
+// on v_mfma_f32_32x32x16_f16 (_bf16 for bf16 activations), activations
+// streamed straight into LDS.
 //
 // Replaces, in function, the reference's large-M routes (paths relative to
 // /root/reference/After-Revision-DROFELL): q4_matmul_cudablas_v2
@@ -33,7 +34,12 @@
 //     unit per 16 lanes) hit 16 different unit positions, conflict-free;
 //   * dequantisation as everywhere in this library: the exact fp16 weight
 //     fp16_rne(s * (q - z)) from the 0x6400 identity, so the product equals
-//     "dequantise, then an fp32-accumulated matmul";
+//     "dequantise, then an fp32-accumulated matmul"; bf16 activations take
+//     bf16_rne(s * (q - z)), one mixed-precision FMA per value and one packed
+//     conversion per pair (17 instead of 13 vector instructions per fragment);
+//   * the 96-row tile is for the row counts between the others: M=384 on 4096
+//     x 11008 takes 172 workgroups of it in one round, 49.0 us, against 129
+//     half-filling ones of 128 rows, 59.0, or 258 of 64 rows, two rounds;
 //   * split-K (several workgroups per tile along K): each split writes its
 //     fp32 partial plane and a second kernel sums the planes in split order
 //     (deterministic) into y.
@@ -58,18 +64,20 @@ __device__ __forceinline__ uint32_t lds_addr(const void* p) {
   return (uint32_t)(uintptr_t)(const lds_void*)p;
 }
 
-// global -> LDS copies: each active lane's 16 (4) bytes at g land at LDS
-// address `lds` + lane * 16 (* 4).  Written as inline assembly so that the
-// compiler's wait-count pass does not track them: it cannot tell which LDS
-// reads such a copy may overlap and would drain every outstanding load
-// before them.  The kernel waits for its copies itself (vmcnt) and makes
-// them visible to the other waves with a barrier.  m0 carries the LDS base
-// (one wait state before its use); nothing else in these kernels uses m0.
-__device__ __forceinline__ void dma16(const void* g, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
-               :: "v"(g), "s"(lds) : "memory");
+// global -> LDS copies: each active lane's 16 (4) bytes at resource base +
+// voff + soff land at LDS address `lds` + lane * 16 (* 4).  Buffer form: the
+// chunk's offset is a scalar, so a copy costs no vector instruction.  Written
+// as inline assembly so that the compiler's wait-count pass does not track
+// them: it cannot tell which LDS reads such a copy may overlap and would
+// drain every outstanding load before them.  The kernel waits for its copies
+// itself (vmcnt) and makes them visible to the other waves with a barrier.
+// m0 carries the LDS base (one wait state before its use); nothing else in
+// these kernels uses m0.
+__device__ __forceinline__ void dma16(uint32_t voff, __amdgpu_buffer_rsrc_t r, int soff, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
+               :: "v"(voff), "s"(r), "s"(soff), "s"(lds) : "memory");
 }
-__device__ __forceinline__ void dma4(const void* g, uint32_t lds) {
+__device__ __forceinline__ void dma4_flat(const void* g, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off"
                :: "v"(g), "s"(lds) : "memory");
 }
@@ -112,27 +120,12 @@ struct Tile {
   static_assert(kStrips % kWaves == 0 && kKS * CG == kWaves, "wave roles cover the tile");
 };
 
-// Matrices of one launch: equal K, N and group size, each with its own
-// packed buffers, bias, output and residual.  Column tile t of the launch
-// belongs to matrix t / ntiles_item (tiles never straddle two matrices).
-struct P2Items {
-  const u4* pq[kGroupMax];
-  const uint32_t* pz[kGroupMax];
-  const uint32_t* ps[kGroupMax];
-  const uint16_t* bias[kGroupMax];
-  uint16_t* y[kGroupMax];
-  int64_t ldy[kGroupMax];
-  const uint16_t* res[kGroupMax];
-  int64_t ldres[kGroupMax];
-  int ntiles_item;
-};
-
 }  // namespace
 
-template <int MTW, int CG, int GPC, int W>
+template <int MTW, int CG, int GPC, int W, bool BF>
 __global__ void __launch_bounds__(W * 64)
 prefill2_kernel(const _Float16* __restrict__ x, int64_t ldx, int M, const P2Items it,
-                float* __restrict__ part, int K, int N, int gs, int G,
+                float* __restrict__ part, int K, int N, uint32_t gmag, int G,
                 int chunks_per_split, int mtiles, int ntiles, int splits, int group_m) {
   using T = Tile<MTW, CG, GPC, W>;
   constexpr int kWaves = W;
@@ -146,25 +139,8 @@ prefill2_kernel(const _Float16* __restrict__ x, int64_t ldx, int M, const P2Item
   static_assert(S >= 2 && S * T::kBytes <= T::kLds, "LDS ring fits the workgroup's share");
   __shared__ __attribute__((aligned(256))) unsigned char ring[S * T::kBytes];
 
-  // XCD-aware order over units (column tile, K split), u = split * ntiles +
-  // ntile: workgroup b runs on XCD b % 8 and takes the XCD's (b / 8)-th
-  // (row tile, unit) pair; XCD x owns the units congruent to x mod 8
-  // (ceil(units / 8) each, the padding ones exit).  On one XCD the pairs
-  // run in groups of group_m row tiles: within a group, the row tiles of
-  // one unit are consecutive, then the next unit's, so the workgroups an
-  // XCD runs at once share both the units' weights and the group's
-  // activation rows in its L2 (group_m = all row tiles: every row tile of
-  // a unit on one XCD in turn).
-  const int b = blockIdx.x;
-  const int nul = (ntiles * splits + 7) / 8;
-  const int pos = b >> 3;  // position in this XCD's order
-  const int grp = pos / (group_m * nul);
-  const int first_m = grp * group_m;
-  const int gsz = min(mtiles - first_m, group_m);
-  const int jj = pos - grp * group_m * nul;
-  const int mtile = first_m + jj % gsz;
-  const int unit = (jj / gsz) * 8 + (b & 7);
-  if (unit >= ntiles * splits) return;
+  int mtile, unit;
+  if (!tile_of(blockIdx.x, mtiles, ntiles * splits, group_m, mtile, unit)) return;
   const int split = unit / ntiles;
   // the launch's column tile -> (matrix, its column tile); wave-uniform
   const int item = (unit % ntiles) / it.ntiles_item;
@@ -201,28 +177,31 @@ prefill2_kernel(const _Float16* __restrict__ x, int64_t ldx, int M, const P2Item
   // activations: copy a of this wave fills units (wave * kAInstr + a) * 64 +
   // lane: row r = unit / 16 at stored position unit % 16, which holds
   // logical unit (unit % 16) ^ (r % 16)
-  const _Float16* asrc[T::kAInstr];
+  const __amdgpu_buffer_rsrc_t ar = rsrc_of(x + (size_t)m0 * ldx + (size_t)c_begin * kChunkK);
+  uint32_t aoff_g[T::kAInstr];
 #pragma unroll
   for (int a = 0; a < T::kAInstr; ++a) {
     const int unit = (wave * T::kAInstr + a) * 64 + lane;
     const int r = unit >> 4;
     const int u = (unit & 15) ^ (r & 15);
-    asrc[a] = x + (size_t)min(m0 + r, M - 1) * ldx + (size_t)c_begin * kChunkK + u * 8;
+    aoff_g[a] = (uint32_t)((min(m0 + r, M - 1) - m0) * (int)ldx + u * 8) * 2;
   }
   // packed weights: tile strip wave * kBInstr + bi, chunk-contiguous (the
-  // last column tile may be partial: missing strips read strip 0, their
-  // columns are not stored)
-  const u4* bsrc[T::kBInstr];
+  // last column tile may be partial: missing strips read the tile's first,
+  // their columns are not stored)
+  const __amdgpu_buffer_rsrc_t br = rsrc_of(pq + ((size_t)strip0 * KC + c_begin) * 64);
+  int bso[T::kBInstr];
 #pragma unroll
   for (int bi = 0; bi < T::kBInstr; ++bi) {
-    const int st = strip0 + wave * T::kBInstr + bi;
-    bsrc[bi] = pq + ((size_t)(st < NS ? st : 0) * KC + c_begin) * 64 + lane;
+    const int st = wave * T::kBInstr + bi;
+    bso[bi] = (strip0 + st < NS ? st : 0) * KC * 1024;
   }
   // scale and zero dwords: dword D of the meta block (D = (mi * 8 + wave) * 64
   // + lane) belongs to column group D / (40 GPC); within it, d < 32 GPC are
   // scales (strip d / (8 GPC), group d / 8 % GPC, word d % 8), then 8 GPC
   // zero words (strip e / (2 GPC), group e / 2 % GPC, word e % 2); dwords
-  // past the block re-read dword 0
+  // past the block re-read dword 0.  Scales and zeros are different buffers,
+  // so a lane's address is a 64-bit one.
   const uint32_t* msrc[T::kMetaInstr];
   int mstride[T::kMetaInstr];
 #pragma unroll
@@ -247,15 +226,15 @@ prefill2_kernel(const _Float16* __restrict__ x, int64_t ldx, int M, const P2Item
     const uint32_t base = ring0 + stage * T::kBytes;
 #pragma unroll
     for (int a = 0; a < T::kAInstr; ++a)
-      dma16(asrc[a] + (size_t)i * kChunkK, base + (wave * T::kAInstr + a) * 1024);
+      dma16(aoff_g[a], ar, i * (kChunkK * 2), base + (wave * T::kAInstr + a) * 1024);
 #pragma unroll
     for (int bi = 0; bi < T::kBInstr; ++bi)
-      dma16(bsrc[bi] + (size_t)i * 64, base + T::kA + (wave * T::kBInstr + bi) * 1024);
+      dma16(lane * 16, br, bso[bi] + i * 1024, base + T::kA + (wave * T::kBInstr + bi) * 1024);
     const int c = c_begin + i;
-    const int g0 = GPC == 1 ? (c * kChunkK) / gs : c * GPC;  // first group of the chunk
+    const int g0 = GPC == 1 ? div_by_magic(c, gmag) : c * GPC;  // first group of the chunk
 #pragma unroll
     for (int mi = 0; mi < T::kMetaInstr; ++mi)
-      dma4(msrc[mi] + (size_t)g0 * mstride[mi], base + T::kA + T::kB + (mi * kWaves + wave) * 256);
+      dma4_flat(msrc[mi] + (size_t)g0 * mstride[mi], base + T::kA + T::kB + (mi * kWaves + wave) * 256);
   };
 
   // ---- LDS offsets (bytes within a stage).  A fragment of k-step t: lane
@@ -298,17 +277,15 @@ prefill2_kernel(const _Float16* __restrict__ x, int64_t ldx, int M, const P2Item
         qw[si][T::kWords - 1] = v.y;
       }
     }
-    h2 nz1024[kPairs][T::kGroups], nz64[kPairs][T::kGroups];
-    _Float16 sc[kPairs][T::kGroups];
+    ColGroup<BF> col[kPairs][T::kGroups];
 #pragma unroll
     for (int p = 0; p < kPairs; ++p)
 #pragma unroll
       for (int gl = 0; gl < T::kGroups; ++gl) {
         const int sl = 2 * p + hi;  // this lane's strip within the column group
         const int g = gbase + gl;
-        zero_consts(meta[32 * GPC + sl * 2 * GPC + g * 2 + (j >> 3)], zsh, nz1024[p][gl],
-                    nz64[p][gl]);
-        sc[p][gl] = as_h((uint16_t)(meta[sl * 8 * GPC + g * 8 + (j >> 1)] >> hsh));
+        col[p][gl].set(meta[sl * 8 * GPC + g * 8 + (j >> 1)], hsh,
+                       meta[32 * GPC + sl * 2 * GPC + g * 2 + (j >> 3)], zsh);
       }
     uint32_t ev[kPairs], od[kPairs];
     auto dequant = [&](int tt, h8 (&bop)[kPairs]) {
@@ -317,9 +294,7 @@ prefill2_kernel(const _Float16* __restrict__ x, int64_t ldx, int M, const P2Item
       for (int p = 0; p < kPairs; ++p) {
         if ((tt & 1) == 0)
           strip_pair_to_b32(qw[2 * p][tt >> 1], qw[2 * p + 1][tt >> 1], ev[p], od[p]);
-        const h8 d = centered8((tt & 1) ? od[p] : ev[p], nz1024[p][gl], nz64[p][gl], magic);
-        const _Float16 s = sc[p][gl];
-        bop[p] = d * h8{s, s, s, s, s, s, s, s};  // fp16 product, round to nearest even
+        bop[p] = weight8((tt & 1) ? od[p] : ev[p], col[p][gl], magic);
       }
     };
     auto read_a = [&](int tt, h8 (&af)[kMT]) {
@@ -339,7 +314,8 @@ prefill2_kernel(const _Float16* __restrict__ x, int64_t ldx, int M, const P2Item
 #pragma unroll
       for (int mt = 0; mt < kMT; ++mt)
 #pragma unroll
-        for (int p = 0; p < kPairs; ++p) acc[mt][p] = mfma32(af[cur][mt], bop[cur][p], acc[mt][p]);
+        for (int p = 0; p < kPairs; ++p)
+          acc[mt][p] = mfma32_of<BF>(af[cur][mt], bop[cur][p], acc[mt][p]);
     }
   };
 
@@ -422,13 +398,13 @@ prefill2_kernel(const _Float16* __restrict__ x, int64_t ldx, int M, const P2Item
   // ---- output: the owners stage the fp16 BM x BN tile in LDS in row
   // order, then all 512 threads store 16-byte row segments
   static_assert(kBM * BN * 2 <= S * T::kBytes, "output tile fits the LDS ring");
-  _Float16* Ts = reinterpret_cast<_Float16*>(ring);
+  uint16_t* Ts = reinterpret_cast<uint16_t*>(ring);
   if (owner) {
-    _Float16 bv[kPairs];
+    uint16_t bv[kPairs];
 #pragma unroll
     for (int p = 0; p < kPairs; ++p) {
       const int st = gstrip0 + 2 * p + hi;
-      bv[p] = (bias != nullptr && st < NS) ? as_h(bias[st * kStripN + j]) : (_Float16)0.f;
+      bv[p] = (bias != nullptr && st < NS) ? bias[st * kStripN + j] : (uint16_t)0;
     }
 #pragma unroll
     for (int mt = 0; mt < kMT; ++mt)
@@ -436,10 +412,8 @@ prefill2_kernel(const _Float16* __restrict__ x, int64_t ldx, int M, const P2Item
       for (int p = 0; p < kPairs; ++p)
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-          _Float16 out = (_Float16)acc[mt][p][i];
-          if (bias != nullptr) out = out + bv[p];
           const int row = mt * 32 + 8 * (i >> 2) + 4 * hb + (i & 3);
-          Ts[row * BN + cg * 64 + p * 32 + l32] = out;
+          Ts[row * BN + cg * 64 + p * 32 + l32] = round_out<BF>(acc[mt][p][i], bias != nullptr, bv[p]);
         }
   }
   __syncthreads();
@@ -478,33 +452,13 @@ prefill2_kernel(const _Float16* __restrict__ x, int64_t ldx, int M, const P2Item
   }
 }
 
-// Row tiles per group of the workgroup order (kernel comment above): all of
-// them up to 8 (a unit's weights then come into an XCD's L2 once), groups of
-// 8 above.  Measured against one group at M=4096 (32 row tiles of 128):
-// 4096^2 144.9 -> 139.6 us, 4096x11008 401.3 -> 391.0, 11008x4096 369.2 ->
-// 353.8; groups of 2 and 4 within 1% of 8; M <= 2048 unchanged.
-constexpr int kPrefillGroupM = 8;
-static int prefill_group_m(int mtiles) { return mtiles <= kPrefillGroupM ? mtiles : kPrefillGroupM; }
-
-template <int MTW, int CG, int GPC, int W>
+template <int MTW, int CG, int GPC, int W, bool BF>
 static hipError_t launch_prefill2_cfg(const GroupArgs& g, int splits, void* ws,
                                       hipStream_t stream) {
   using T = Tile<MTW, CG, GPC, W>;
   const GemmArgs& a = g.a[0];
   const int mtiles = (a.M + T::kBM - 1) / T::kBM;
-  P2Items it{};
-  it.ntiles_item = (a.N + T::kBN - 1) / T::kBN;
-  for (int i = 0; i < kGroupMax; ++i) {
-    const GemmArgs& b = g.a[i < g.count ? i : 0];
-    it.pq[i] = reinterpret_cast<const u4*>(b.pq);
-    it.pz[i] = b.pz;
-    it.ps[i] = reinterpret_cast<const uint32_t*>(b.ps);
-    it.bias[i] = b.bias;
-    it.y[i] = b.y;
-    it.ldy[i] = b.ldy;
-    it.res[i] = b.res;
-    it.ldres[i] = b.ldres;
-  }
+  const P2Items it = prefill_items(g, T::kBN);
   const int ntiles = it.ntiles_item * g.count;
   const int KC = a.K / kChunkK;
   const int cps = (KC + splits - 1) / splits;
@@ -514,51 +468,45 @@ static hipError_t launch_prefill2_cfg(const GroupArgs& g, int splits, void* ws,
                     ? reinterpret_cast<float*>(static_cast<unsigned char*>(ws) + kWsHeadBytes)
                     : nullptr;
   const int units = ntiles * real_splits;
-  const dim3 grid((unsigned)(((units + 7) / 8) * 8 * mtiles));
-  prefill2_kernel<MTW, CG, GPC, W><<<grid, W * 64, 0, stream>>>(
-      (const _Float16*)a.x, a.ldx, a.M, it, part, a.K, a.N, a.gs, a.G, cps, mtiles, ntiles,
-      real_splits, prefill_group_m(mtiles));
+  const dim3 grid((unsigned)((units * mtiles + 7) / 8 * 8));
+  prefill2_kernel<MTW, CG, GPC, W, BF><<<grid, W * 64, 0, stream>>>(
+      (const _Float16*)a.x, a.ldx, a.M, it, part, a.K, a.N, group_magic(a.gs), a.G, cps, mtiles,
+      ntiles, real_splits, prefill_group_m(mtiles));
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess || real_splits == 1) return e;
   return launch_reduce_planes(part, real_splits, a.M, a.N, a.bias, a.y, a.ldy, a.res, a.ldres,
-                              stream);
+                              stream, BF);
+}
+
+template <int MTW, int CG, int W, bool BF>
+static hipError_t launch_prefill2_gpc(const GroupArgs& a, int splits, void* ws,
+                                      hipStream_t stream) {
+  const int gpc = a.a[0].gs >= kChunkK ? 1 : kChunkK / a.a[0].gs;
+  if (gpc == 1) return launch_prefill2_cfg<MTW, CG, 1, W, BF>(a, splits, ws, stream);
+  if (gpc == 2) return launch_prefill2_cfg<MTW, CG, 2, W, BF>(a, splits, ws, stream);
+  return launch_prefill2_cfg<MTW, CG, 4, W, BF>(a, splits, ws, stream);
 }
 
 template <int MTW, int CG, int W>
-static hipError_t launch_prefill2_tile(const GroupArgs& a, int splits, void* ws,
+static hipError_t launch_prefill2_tile(const GroupArgs& a, const PrefillPlan& p, void* ws,
                                        hipStream_t stream) {
-  const int gpc = a.a[0].gs >= kChunkK ? 1 : kChunkK / a.a[0].gs;
-  if (gpc == 1) return launch_prefill2_cfg<MTW, CG, 1, W>(a, splits, ws, stream);
-  if (gpc == 2) return launch_prefill2_cfg<MTW, CG, 2, W>(a, splits, ws, stream);
-  return launch_prefill2_cfg<MTW, CG, 4, W>(a, splits, ws, stream);
-}
-
-hipError_t launch_prefill2(const GemmArgs& one, const PrefillPlan& plan, void* ws,
-                           hipStream_t stream) {
-  GroupArgs g{};
-  g.count = 1;
-  g.a[0] = one;
-  return launch_prefill2_group(g, plan, ws, stream);
+  if (p.bf16) return launch_prefill2_gpc<MTW, CG, W, true>(a, p.splits, ws, stream);
+  return launch_prefill2_gpc<MTW, CG, W, false>(a, p.splits, ws, stream);
 }
 
 hipError_t launch_prefill2_group(const GroupArgs& a, const PrefillPlan& plan, void* ws,
                                  hipStream_t stream) {
-  if (a.count < 1 || a.count > kGroupMax) return hipErrorInvalidValue;
-  for (int i = 0; i < a.count; ++i) {
-    const GemmArgs& b = a.a[i];
-    // x must already be in packed row order; one x, K, N and group size
-    if (b.perm != nullptr || b.x != a.a[0].x || b.ldx != a.a[0].ldx || b.M != a.a[0].M ||
-        b.K != a.a[0].K || b.N != a.a[0].N || b.gs != a.a[0].gs)
-      return hipErrorInvalidValue;
-  }
+  if (!same_x_shape(a) || !prefill_x_fits(a.a[0].ldx)) return hipErrorInvalidValue;
+  if (plan.bf16 && a.a[0].res != nullptr) return hipErrorInvalidValue;
   if (plan.waves == 4) {  // two workgroups per CU
-    if (plan.bm == 64 && plan.bn == 128) return launch_prefill2_tile<2, 2, 4>(a, plan.splits, ws, stream);
-    if (plan.bm == 32 && plan.bn == 128) return launch_prefill2_tile<1, 2, 4>(a, plan.splits, ws, stream);
+    if (plan.bm == 64 && plan.bn == 128) return launch_prefill2_tile<2, 2, 4>(a, plan, ws, stream);
+    if (plan.bm == 32 && plan.bn == 128) return launch_prefill2_tile<1, 2, 4>(a, plan, ws, stream);
     return hipErrorInvalidValue;
   }
-  if (plan.bm == 64 && plan.bn == 256) return launch_prefill2_tile<2, 4, 8>(a, plan.splits, ws, stream);
-  if (plan.bm == 128 && plan.bn == 256) return launch_prefill2_tile<4, 4, 8>(a, plan.splits, ws, stream);
-  if (plan.bm == 128 && plan.bn == 128) return launch_prefill2_tile<4, 2, 8>(a, plan.splits, ws, stream);
+  if (plan.bm == 64 && plan.bn == 256) return launch_prefill2_tile<2, 4, 8>(a, plan, ws, stream);
+  if (plan.bm == 96 && plan.bn == 256) return launch_prefill2_tile<3, 4, 8>(a, plan, ws, stream);
+  if (plan.bm == 128 && plan.bn == 256) return launch_prefill2_tile<4, 4, 8>(a, plan, ws, stream);
+  if (plan.bm == 128 && plan.bn == 128) return launch_prefill2_tile<4, 2, 8>(a, plan, ws, stream);
   return hipErrorInvalidValue;
 }
 
