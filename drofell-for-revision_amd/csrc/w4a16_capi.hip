@@ -593,6 +593,58 @@ int dw4_gemm_bf16(int m, int k, int n, int group_size, const uint16_t* x, int64_
   return status_of(dw4::launch_decode_reg_bf16(a, dw4::plan_decode_bf16(m, k, n, group_size, cu_count()), s));
 }
 
+int dw4_gemm_bf16_prefill(int m, int k, int n, int group_size, const uint16_t* x, int64_t ldx,
+                          const int32_t* packed_qweight, const int32_t* packed_zeros,
+                          const uint16_t* packed_scales, const int32_t* perm,
+                          const uint16_t* bias, uint16_t* y, int64_t ldy, void* workspace,
+                          size_t workspace_bytes, void* stream) {
+  const int st = check_shape(k, n, group_size);
+  if (st != DW4_OK) return st;
+  if (m < 0) return DW4_ERR_INVALID_ARG;
+  if (m == 0) return DW4_OK;
+  if (!x || !packed_qweight || !packed_zeros || !packed_scales || !y) return DW4_ERR_INVALID_ARG;
+  if (ldx < k || ldy < n) return DW4_ERR_INVALID_ARG;
+  if (!aligned16(x) || (ldx % 8) != 0 || !aligned16(packed_qweight)) return DW4_ERR_MISALIGNED;
+  if (perm == nullptr && !dw4::prefill_x_fits(ldx)) return DW4_ERR_UNSUPPORTED;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const size_t room = workspace && aligned16(workspace) ? workspace_bytes : 0;
+  // act-order: the gathered rows (2-byte elements: the fp16 gather serves
+  // bf16) after the planes; the kernels do not gather themselves
+  const size_t gather = perm != nullptr ? dw4::gather_bytes(m, k) : 0;
+  if (perm != nullptr && room < dw4::gather_offset(0) + gather) return DW4_ERR_WORKSPACE;
+  // (whole 256 bytes, as gather_offset aligns the rows after the planes)
+  dw4::PrefillPlan plan =
+      plan_stream(m, k, n, 1, 0, room > gather ? (room - gather) & ~(size_t)255 : 0);
+  plan.bf16 = true;
+  dw4::GroupArgs g{};
+  g.count = 1;
+  dw4::GemmArgs& a = g.a[0];
+  a.M = m;
+  a.K = k;
+  a.N = n;
+  a.gs = group_size;
+  a.G = k / group_size;
+  a.x = x;
+  a.ldx = ldx;
+  a.pq = reinterpret_cast<const uint32_t*>(packed_qweight);
+  a.pz = reinterpret_cast<const uint32_t*>(packed_zeros);
+  a.ps = packed_scales;
+  a.perm = nullptr;
+  a.bias = bias;
+  a.y = y;
+  a.ldy = ldy;
+  if (perm != nullptr) {
+    const size_t off =
+        dw4::gather_offset(plan.splits > 1 ? stream_ws_bytes(plan.splits, m, n) : 0);
+    uint16_t* xs = reinterpret_cast<uint16_t*>(static_cast<unsigned char*>(workspace) + off);
+    const int e = status_of(dw4::launch_gather_rows(x, ldx, perm, xs, k, m, s));
+    if (e != DW4_OK) return e;
+    a.x = xs;
+    a.ldx = k;
+  }
+  return status_of(launch_stream(g, plan, workspace, s));
+}
+
 int dw4_dequant(int k, int n, int group_size, const int32_t* packed_qweight,
                 const int32_t* packed_zeros, const uint16_t* packed_scales, const int32_t* perm,
                 uint16_t* w, int64_t ldw, void* stream) {

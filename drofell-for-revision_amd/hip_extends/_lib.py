@@ -80,6 +80,8 @@ SIGNATURES = {
                             _P, _P, _P, _P, _P, _P, _c.c_int64, _P, _c.c_size_t, _P]),
     "dw4_gemm_bf16": (_c.c_int, [_c.c_int, _c.c_int, _c.c_int, _c.c_int, _P, _c.c_int64,
                                  _P, _P, _P, _P, _P, _P, _c.c_int64, _P, _c.c_size_t, _P]),
+    "dw4_gemm_bf16_prefill": (_c.c_int, [_c.c_int, _c.c_int, _c.c_int, _c.c_int, _P, _c.c_int64,
+                                         _P, _P, _P, _P, _P, _P, _c.c_int64, _P, _c.c_size_t, _P]),
     "dw4_gemm_path": (_c.c_int, [_c.c_int, _c.c_int, _c.c_int, _c.c_int, _c.c_int, _c.c_int,
                                  _P, _c.c_int64, _P, _P, _P, _P, _P, _P, _c.c_int64,
                                  _P, _c.c_size_t, _P]),
@@ -128,6 +130,12 @@ SIGNATURES = {
 }
 ABI_VERSION = 11
 BF16_MAX_M = 64  # DW4_BF16_MAX_M
+# Rows up to which bf16 x runs on the packed words (prefill kernels) rather
+# than over a dequantised weight (us, packed against dequantise + library GEMM):
+# M=65 4096^2 14.0 / 37.6, M=256 11008x4096 38.4 / 90.2, M=700 4096x11008 90.0 /
+# 110.6, M=1024 5120x13824 153 / 159, M=1536 235 / 237 there and 152 / 166 at
+# 11008x4096; at M=2048 315 / 284, at M=3072 the dense route wins on every shape.
+BF16_PREFILL_MAX_M = 1536
 
 _lock = threading.Lock()
 _lib: Optional[ctypes.CDLL] = None

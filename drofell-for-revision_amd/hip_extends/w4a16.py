@@ -342,15 +342,17 @@ class Q4MatrixV2(object):
           library GEMM); otherwise the HIP W4A16 kernel (decode kernel for
           small M, MFMA prefill kernel above);
         * bf16 x: with a reconstructed bf16 weight, ``must_blas`` or more
-          than ``BF16_MAX_M`` rows, the dense bf16 product (fp32
+          than ``BF16_PREFILL_MAX_M`` rows, the dense bf16 product (fp32
           accumulation) over the bf16 weight bf16(fp16(s * (q - z))), the
           reconstructed one or one dequantised into ``temp_weight`` / the
           shared buffer, as the reference's ``q4_matmul_blas_v2`` with
           ``bfloat16`` does; up to ``BF16_MAX_M`` rows the HIP decode
           kernel's bf16 mode (``dw4_gemm_bf16``: bf16 matrix cores over the
           packed words, the exact s * (q - z) applied per group in fp32, bf16
-          output, one launch), within rounding of the dense product.  The
-          activations keep bf16's range either way.
+          output, one launch), between the two the HIP prefill kernels
+          (``dw4_gemm_bf16_prefill``: the weight rounded once to bf16 in the
+          kernel), within rounding of the dense product.  The activations
+          keep bf16's range either way.
 
         ``output`` (x's dtype, ``M * N`` elements, contiguous or a row-strided
         [M, N] view) receives the product; anything else raises.  ``bias``
@@ -370,17 +372,24 @@ class Q4MatrixV2(object):
             bias = bias.to(dtype).contiguous()
         dense = self._reconstructed(dtype)
         if dtype == torch.bfloat16 and dense is None and not must_blas \
-                and 0 < m <= _lib.BF16_MAX_M:
+                and 0 < m <= _lib.BF16_PREFILL_MAX_M:
+            fn = "dw4_gemm_bf16" if m <= _lib.BF16_MAX_M else "dw4_gemm_bf16_prefill"
             x2 = _aligned_rows(x.reshape(m, self.height))
-            if out2 is None:
-                out2 = torch.empty((m, self.width), dtype=torch.bfloat16, device=self.device)
+            y2 = torch.empty((m, self.width), dtype=torch.bfloat16, device=self.device) \
+                if out2 is None else out2
             ws = self.cache.workspace
-            _lib.check("dw4_gemm_bf16", _lib.load().dw4_gemm_bf16(
+            status = getattr(_lib.load(), fn)(
                 m, self.height, self.width, self.group_size, x2.data_ptr(), x2.stride(0),
                 self.qweight.data_ptr(), self.qzeros.data_ptr(), self.scales.data_ptr(),
                 _ptr(self.perm) if self.use_act else None, _ptr(bias),
-                out2.data_ptr(), out2.stride(0), ws.data_ptr(), ws.numel(), _stream(self.device)))
-            return out2.view(outshape) if output is None else output
+                y2.data_ptr(), y2.stride(0), ws.data_ptr(), ws.numel(), _stream(self.device))
+            # the prefill kernels do not take act-order calls whose workspace
+            # cannot hold the gathered rows, nor very wide row strides: those
+            # keep the dense route (nothing was launched)
+            if m <= _lib.BF16_MAX_M or status not in (_lib.DW4_ERR_WORKSPACE,
+                                                      _lib.DW4_ERR_UNSUPPORTED):
+                _lib.check(fn, status)
+                return y2.view(outshape) if output is None else output
         if dense is not None or must_blas or dtype == torch.bfloat16:
             w = dense if dense is not None else self._dense_weight(temp_weight, dtype)
             x2 = x.reshape(m, self.height)

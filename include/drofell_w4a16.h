@@ -192,6 +192,21 @@ int dw4_gemm_bf16(int m, int k, int n, int group_size,
                   const uint16_t* bias, uint16_t* y, int64_t ldy,
                   void* workspace, size_t workspace_bytes, void* stream);
 
+/* Device: the same product for any m >= 1 on the prefill kernels (bf16 matrix
+ * cores, the packed words dequantised in the kernel to bf16(s (q - z)), rounded
+ * once; fp32 accumulation).  Buffers, alignment, bias and output as in
+ * dw4_gemm_bf16.  A K split uses the workspace's planes where they fit.
+ * Act-order calls need room for the gathered rows (dw4_workspace_size(m, ...,
+ * act_order = 1) bytes, zero-filled once) and return DW4_ERR_WORKSPACE without;
+ * row strides of x beyond 2^22 elements return DW4_ERR_UNSUPPORTED (x without
+ * a perm).  Meant for m > DW4_BF16_MAX_M. */
+int dw4_gemm_bf16_prefill(int m, int k, int n, int group_size,
+                          const uint16_t* x, int64_t ldx,
+                          const int32_t* packed_qweight, const int32_t* packed_zeros,
+                          const uint16_t* packed_scales, const int32_t* perm,
+                          const uint16_t* bias, uint16_t* y, int64_t ldy,
+                          void* workspace, size_t workspace_bytes, void* stream);
+
 /* dw4_gemm with an explicit path (DW4_PATH_*) and prefill split-K factor
  * (0 = automatic); for tests and benchmarks. */
 int dw4_gemm_path(int path, int split_k, int m, int k, int n, int group_size,
