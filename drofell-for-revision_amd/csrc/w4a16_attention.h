@@ -8,7 +8,9 @@
 namespace dw4 {
 
 // Paged-attention decode over the block pointer tables of a KV cache.
-constexpr int kAttnMaxPartTokens = 512;  // tokens per context partition, at most
+// Tokens per context partition with grouped heads, at most: a lane holds the address of one block
+// of its wave, 64 blocks of 16 tokens per wave and four waves.
+constexpr int kAttnMaxPartTokens = 4096;
 constexpr int kAttnMaxGroup = 8;         // query heads per kv head, at most
 struct PagedAttnArgs {
   int num_seqs, num_heads, num_kv_heads, head_size, block_size;
@@ -28,21 +30,22 @@ struct PagedAttnArgs {
 struct PagedAttnPlan {
   int part_tokens = kAttnMaxPartTokens;
   int num_parts = 1;
-  int waves = 4;  // per workgroup: 4, or 16 for one workgroup per (sequence, kv head)
+  int waves = 4;  // per workgroup: 4, or 8 (one head per kv head: 16) for one workgroup per
+                  // (sequence, kv head)
 };
-// The 16-wave form: contexts up to this many tokens in one partition, for
-// the (head size, block size, query-head group) variants whose per-wave
-// partial outputs fit LDS and whose registers fit 1024-thread workgroups.
-constexpr int kAttnWideMaxTokens = 1024;
-constexpr bool attn_wide_ok(int hs, int bs, int gmax) {
-  return bs == 16 && hs <= 128 && gmax * hs <= 512;
+// The 8-wave form: contexts up to this many tokens in one partition.
+constexpr int kAttnWideMaxTokens = 4096;
+// Dynamic LDS of a paged-attention workgroup: the waves' outputs
+// [waves][g][hs] and their max and sum per head.
+inline size_t attn_smem_bytes(int hs, int g, int waves) {
+  return sizeof(float) * (size_t)waves * g * (hs + 2);
 }
-// Dynamic LDS of a paged-attention workgroup: the scaled queries [gmax][hs],
-// the logits [gmax][part_tokens], the waves' partial outputs
-// [waves][gmax][hs] and one float per wave for block reductions.
-inline size_t attn_smem_bytes(int hs, int gmax, int part_tokens, int waves) {
-  return sizeof(float) * ((size_t)gmax * hs + (size_t)gmax * part_tokens +
-                          (size_t)waves * gmax * hs + waves);
+// One query head per kv head: partitions of up to 512 tokens, or the 16-wave
+// form's one of up to 1024; dynamic LDS for the scaled query [hs], the logits
+// [part_tokens], the waves' outputs [waves][hs] and one float per wave.
+constexpr int kAttnRowPartTokens = 512, kAttnRowWideTokens = 1024;
+inline size_t attn_row_smem_bytes(int hs, int part_tokens, int waves) {
+  return sizeof(float) * ((size_t)hs + part_tokens + (size_t)waves * hs + waves);
 }
 PagedAttnPlan plan_paged_attention(int num_seqs, int num_heads, int num_kv_heads, int head_size,
                                    int block_size, int max_context_len, int cus);

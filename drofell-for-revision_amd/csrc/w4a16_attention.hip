@@ -12,15 +12,31 @@
 // paged_attention_kernel: one workgroup per (sequence, kv head, context
 // partition).  It serves every query head of the kv head's group
 // (head h uses kv head h / (heads / kv_heads)), so each K and V byte is
-// read once per group.  Per partition of up to 512 tokens:
-//   logits (fp32, LDS) = scale * q . k (+ alibi slope * (t - ctx + 1));
+// read once per group.  Per partition of up to 4096 tokens:
+//   logits = scale * q . k (+ alibi slope * (t - ctx + 1));
 //   p = exp(logit - max); out = sum p v / sum p.
-// Waves take the partition's blocks round-robin.  For q . k a lane holds one
-// token and a slice of 8 dims (one 16-byte load); lanes of one token meet
-// through cross-lane adds.  For p . v a lane holds whole dims (a row of BS
-// tokens).  Partitions write their max, sum and unnormalised fp32 output;
-// a second kernel combines them in partition order (deterministic).  With a
-// single partition the first kernel writes the output directly.
+// HBM-bound (the KV stream), so with grouped heads both products run on the
+// matrix cores, whose
+// operand layouts the cache's already are: the rows of a 16x16x32 MFMA are 16
+// tokens (q . k) or 16 dims (p . v), each lane's 8 reduction elements one
+// 16-byte unit of the cache, loaded straight into the operand registers; the
+// columns are the group's heads (2 to 8 of 16).  A wave takes steps of 32
+// tokens and keeps a running max, sum and output per head (all of head c in
+// the lanes of column c), so no logits go through LDS; with row r of q . k's
+// two token tiles holding tokens 8 (r / 4) + r % 4 and 4 more, a lane's eight
+// logits are those of 8 consecutive tokens, the very p . v operand.
+// Measured (us, with the products on the vector ALU, one LDS read of a logit
+// per p . v FMA, before): 24 x 3000 tokens, 32 heads on 8 of 128 85 -> 46 (4.8
+// TB/s), 32 x 4000, 64 on 8 283 -> 81, 8 x 600, 32 heads 20.5 -> 15.7, 8 x 3000, 16
+// heads of 256 123 -> 54.
+// Precision: q . k sums exact fp16 products in fp32; the softmax and its sums
+// stay in fp32, and p enters p . v as two fp16 parts of 2^14 p (21 bits; what
+// small p lose is below 2^-37 of the largest).
+// Waves take the partition's steps round-robin and meet once in LDS.
+// Partitions write their max, sum and unnormalised fp32 output; a second
+// kernel combines them in partition order (deterministic).  With a single
+// partition the first kernel writes the output directly.  One query head per
+// kv head goes to paged_attention_row_kernel, in partitions of up to 512 tokens.
 
 #include <hip/hip_runtime.h>
 
@@ -34,6 +50,11 @@ namespace dw4 {
 
 namespace {
 
+
+constexpr float kLog2e = 1.4426950408889634f;
+constexpr float kPScale = 16384.f;  // p enters p . v as fp16 parts of 2^14 p
+
+__device__ __forceinline__ float exp_of(float v) { return __builtin_amdgcn_exp2f(v * kLog2e); }
 
 __device__ __forceinline__ float wave_max(float v) {
 #pragma unroll
@@ -61,19 +82,29 @@ __device__ __forceinline__ float block_reduce(float v, float* scratch) {
   return r;
 }
 
-// W waves per workgroup: 4 (several partitions per (sequence, kv head),
-// about four workgroups per CU) or 16 (one workgroup per (sequence, kv head)
-// covering the whole context, no combine launch).
-template <int HS, int BS, int GMAX, int W>
+// The form for one query head per kv head, on the vector ALU: the matrix
+// form's 16 columns would hold one head.  For q . k a lane holds one token and
+// a slice of 8 dims (one 16-byte load), lanes of one token meet through
+// cross-lane adds, the logits stand in LDS; for p . v a lane holds whole dims (a
+// row of BS tokens).  Measured: four layers of 8 x 600 tokens, 32 heads of 128,
+// 283 -> 270 us when this form took one head at compile time instead of a
+// group's; the matrix form 269.  As that gains nothing, this one's order of sums
+// stays: a stack of layers turns single roundings of one layer into
+// differences of whole percents in a later one (an RMS norm over a row whose
+// residuals cancel).
+// W waves per workgroup: 4 (several partitions per (sequence, head), about four
+// workgroups per CU) or 16 (one workgroup per (sequence, head) covering the
+// whole context, no combine launch).
+template <int HS, int BS, int W>
 __global__ void __launch_bounds__(W * 64)
-paged_attention_kernel(const uint16_t* __restrict__ query, int64_t q_stride,
-                       uint16_t* __restrict__ out, int64_t o_stride,
-                       const int64_t* __restrict__ kptr, const int64_t* __restrict__ vptr,
-                       int kv_head_stride, int num_heads, int num_kv_heads, float scale,
-                       const int32_t* __restrict__ block_tables, int max_blocks,
-                       const int32_t* __restrict__ context_lens,
-                       const float* __restrict__ alibi, int part_tokens, int num_parts,
-                       float* __restrict__ ws_ml, float* __restrict__ ws_out) {
+paged_attention_row_kernel(const uint16_t* __restrict__ query, int64_t q_stride,
+                           uint16_t* __restrict__ out, int64_t o_stride,
+                           const int64_t* __restrict__ kptr, const int64_t* __restrict__ vptr,
+                           int kv_head_stride, int num_heads, float scale,
+                           const int32_t* __restrict__ block_tables, int max_blocks,
+                           const int32_t* __restrict__ context_lens,
+                           const float* __restrict__ alibi, int part_tokens, int num_parts,
+                           float* __restrict__ ws_ml, float* __restrict__ ws_out) {
   constexpr int SLICES = HS / 8;                 // 16-byte slices of a key row
   constexpr int TPL = 64 / BS;                   // slice groups per wave (lanes of one token)
   constexpr int SPL = (SLICES + TPL - 1) / TPL;  // slices per lane (the last may be past HS)
@@ -83,11 +114,201 @@ paged_attention_kernel(const uint16_t* __restrict__ query, int64_t q_stride,
   constexpr bool KTAIL = SLICES % TPL != 0, VTAIL = HS % 64 != 0;
   static_assert(HS % 8 == 0 && 64 % BS == 0, "shape");
   extern __shared__ __attribute__((aligned(16))) float sm[];
-  const int G = num_heads / num_kv_heads;  // query heads per kv head (<= GMAX)
-  float* qs = sm;                           // [G][HS] fp32 query (scaled)
-  float* logit = qs + GMAX * HS;            // [G][part_tokens]
-  float* red = logit + GMAX * part_tokens;  // [waves][G][HS] partial outputs
-  float* scratch = red + W * GMAX * HS;  // W floats
+  float* qs = sm;                               // [HS] fp32 query (scaled)
+  float* logit = qs + HS;                   // [part_tokens]
+  float* red = logit + part_tokens;         // [waves][HS] partial outputs
+  float* scratch = red + W * HS;            // W floats
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int seq = blockIdx.x / num_heads;
+  const int head = blockIdx.x % num_heads;
+  const int part = blockIdx.y;
+  // a context longer than the block table is cut to it (never read past a row)
+  const int ctx = min(context_lens[seq], max_blocks * BS);
+  const int t0 = part * part_tokens;
+  const int t1 = min(ctx, t0 + part_tokens);
+  const int nt = t1 - t0;
+  const bool direct = num_parts == 1;
+  if (nt <= 0) {  // partition past this sequence's context: an empty partial
+    if (!direct && tid == 0) {
+      const size_t r = ((size_t)seq * num_heads + head) * num_parts + part;
+      ws_ml[2 * r] = -FLT_MAX;
+      ws_ml[2 * r + 1] = 0.f;
+    }
+    return;
+  }
+  const int32_t* btab = block_tables + (size_t)seq * max_blocks + t0 / BS;
+  const int nb = (nt + BS - 1) / BS;
+  const int nbw = wave < nb ? (nb - wave + W - 1) / W : 0;  // this wave's blocks
+  const int tt = lane % BS;   // token of this lane within a block
+  const int sg = lane / BS;   // slice group
+  // Each wave keeps its next NPF blocks' keys and values in flight: the
+  // value loads of the first blocks are issued with the key loads, before
+  // the softmax, so their latency overlaps q . k.
+  constexpr int NPF = 2;
+  h8 kreg[NPF][SPL];
+  h8 vreg[NPF][DPL][BS / 8];
+  auto kbase = [&](int i) {
+    return reinterpret_cast<const uint16_t*>(kptr[btab[wave + W * i]]) +
+           (size_t)head * kv_head_stride;
+  };
+  auto vbase = [&](int i) {
+    return reinterpret_cast<const uint16_t*>(vptr[btab[wave + W * i]]) +
+           (size_t)head * kv_head_stride;
+  };
+  auto load_k = [&](int slot, int i) {
+    const uint16_t* kb = kbase(i);
+#pragma unroll
+    for (int j = 0; j < SPL; ++j) {
+      if (KTAIL && sg + TPL * j >= SLICES) {
+        kreg[slot][j] = h8{};
+        continue;
+      }
+      kreg[slot][j] = *(const h8*)(kb + ((sg + TPL * j) * BS + tt) * 8);
+    }
+  };
+  auto load_v = [&](int slot, int i) {
+    const uint16_t* vb = vbase(i);
+#pragma unroll
+    for (int j = 0; j < DPL; ++j)
+#pragma unroll
+      for (int u = 0; u < BS / 8; ++u)
+        vreg[slot][j][u] = VTAIL && lane + 64 * j >= HS
+                                   ? h8{}
+                                   : *(const h8*)(vb + (size_t)(lane + 64 * j) * BS + 8 * u);
+  };
+#pragma unroll
+  for (int u = 0; u < NPF; ++u)
+    if (u < nbw) {
+      load_k(u, u);
+      load_v(u, u);
+    }
+  // The query is staged after the first blocks' key and value loads went
+  // out (each behind its block-table and block-pointer loads), so its own
+  // load overlaps theirs; the barrier that publishes it waits only for the
+  // LDS stores, and the key/value loads stay in flight across it (a
+  // __syncthreads would wait for them).
+  for (int d = tid; d < HS; d += (W * 64))
+    qs[d] = scale * (float)as_h(query[(size_t)seq * q_stride + (size_t)head * HS + d]);
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+
+  // q . k
+  auto qk = [&](int slot, int i) {
+    const int b = wave + W * i;
+    float dot = 0.f;
+#pragma unroll
+    for (int j = 0; j < SPL; ++j) {
+      if (KTAIL && sg + TPL * j >= SLICES) continue;
+      const float* qv = qs + (sg + TPL * j) * 8;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) dot = fmaf(qv[e], (float)kreg[slot][j][e], dot);
+    }
+#pragma unroll
+    for (int off = BS; off < 64; off <<= 1) dot += __shfl_xor(dot, off);
+    const int t = t0 + b * BS + tt;
+    if (sg == 0) {
+      if (alibi != nullptr) dot += alibi[head] * (float)(t - ctx + 1);
+      logit[b * BS + tt] = t < t1 ? dot : -FLT_MAX;
+    }
+  };
+  for (int i0 = 0; i0 < nbw; i0 += NPF) {
+#pragma unroll
+    for (int u = 0; u < NPF; ++u) {
+      const int i = i0 + u;
+      if (i < nbw) {
+        qk(u, i);
+        if (i + NPF < nbw) load_k(u, i + NPF);
+      }
+    }
+  }
+  __syncthreads();
+
+  // softmax numerators and their sum
+  float mx = -FLT_MAX, sum = 0.f;
+  for (int t = tid; t < nt; t += (W * 64)) mx = fmaxf(mx, logit[t]);
+  mx = block_reduce<true, W>(mx, scratch);
+  for (int t = tid; t < nb * BS; t += (W * 64)) {
+    const float p = t < nt ? __expf(logit[t] - mx) : 0.f;
+    logit[t] = p;
+    sum += p;
+  }
+  sum = block_reduce<false, W>(sum, scratch);
+  __syncthreads();
+
+  // p . v: lane holds dims lane + 64 j
+  float acc[DPL];
+#pragma unroll
+  for (int j = 0; j < DPL; ++j) acc[j] = 0.f;
+  auto pv = [&](int slot, int i) {
+    const int b = wave + W * i;
+    const int valid = min(BS, nt - b * BS);  // tokens of this block in the context
+#pragma unroll
+    for (int j = 0; j < DPL; ++j)
+#pragma unroll
+      for (int u = 0; u < BS / 8; ++u)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int tb = 8 * u + e;
+          // slots past the context may hold anything: never multiply them
+          const float vf = tb < valid ? (float)vreg[slot][j][u][e] : 0.f;
+          acc[j] = fmaf(logit[b * BS + tb], vf, acc[j]);
+        }
+  };
+  for (int i0 = 0; i0 < nbw; i0 += NPF) {
+#pragma unroll
+    for (int u = 0; u < NPF; ++u) {
+      const int i = i0 + u;
+      if (i < nbw) {
+        pv(u, i);
+        if (i + NPF < nbw) load_v(u, i + NPF);
+      }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < DPL; ++j)
+    if (!VTAIL || lane + 64 * j < HS) red[wave * HS + lane + 64 * j] = acc[j];
+  __syncthreads();
+  for (int d = tid; d < HS; d += (W * 64)) {
+    float o = 0.f;
+#pragma unroll
+    for (int w = 0; w < W; ++w) o += red[w * HS + d];
+    if (direct) {
+      out[(size_t)seq * o_stride + (size_t)head * HS + d] = h_bits((_Float16)(o / sum));
+    } else {
+      const size_t r = ((size_t)seq * num_heads + head) * num_parts + part;
+      ws_out[r * HS + d] = o;
+      if (d == 0) {
+        ws_ml[2 * r] = mx;
+        ws_ml[2 * r + 1] = sum;
+      }
+    }
+  }
+}
+
+// W waves per workgroup: 4 (several partitions per (sequence, kv head)) or 8
+// (one workgroup per (sequence, kv head) covering the whole context, no
+// combine launch).
+template <int HS, int BS, int W>
+__global__ void __launch_bounds__(W * 64, HS <= 128 ? 2 : 1)  // 256 registers per lane, or 512
+paged_attention_kernel(const uint16_t* __restrict__ query, int64_t q_stride,
+                       uint16_t* __restrict__ out, int64_t o_stride,
+                       const int64_t* __restrict__ kptr, const int64_t* __restrict__ vptr,
+                       int kv_head_stride, int num_heads, int num_kv_heads, float scale,
+                       const int32_t* __restrict__ block_tables, int max_blocks,
+                       const int32_t* __restrict__ context_lens,
+                       const float* __restrict__ alibi, int part_tokens, int num_parts,
+                       float* __restrict__ ws_ml, float* __restrict__ ws_out) {
+  constexpr int SLICES = HS / 8;        // 16-byte units of a key row
+  constexpr int NK = (HS + 31) / 32;    // 32-dim reduction steps of q . k (the last may be partial)
+  constexpr int ND = HS / 16;           // 16-dim tiles of p . v
+  constexpr int NB = 32 / BS;           // blocks of a 32-token step
+  constexpr int SLOTS = HS <= 128 ? 2 : 1;  // steps in flight per wave (registers)
+  static_assert(HS % 16 == 0 && 32 % BS == 0, "shape");
+  extern __shared__ __attribute__((aligned(16))) float sm[];
+  const int G = num_heads / num_kv_heads;  // query heads per kv head (<= kAttnMaxGroup)
+  float* red = sm;                          // [waves][G][HS] outputs
+  float* ml = red + W * G * HS;             // [waves][G][2] max, sum
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -109,187 +330,182 @@ paged_attention_kernel(const uint16_t* __restrict__ query, int64_t q_stride,
     }
     return;
   }
-  const int32_t* btab = block_tables + (size_t)seq * max_blocks + t0 / BS;
+  const int c = lane & 15;   // operand row (token, dim) or column (head)
+  const int qd = lane >> 4;  // 8-element group of the reduction
   const int nb = (nt + BS - 1) / BS;
-  const int nbw = wave < nb ? (nb - wave + W - 1) / W : 0;  // this wave's blocks
-  const int tt = lane % BS;   // token of this lane within a block
-  const int sg = lane / BS;   // slice group
-  // Each wave keeps its next NPF blocks' keys and values in flight: the
-  // value loads of the first blocks are issued with the key loads, before
-  // the softmax, so their latency overlaps q . k.
-  // (one block for the widest variants, whose unrolled p . v would not fit)
-  constexpr int NPF = DPL * (BS / 8) * GMAX <= 16 ? 2 : 1;
-  h8 kreg[NPF][SPL];
-  h8 vreg[NPF][DPL][BS / 8];
-  auto kbase = [&](int i) {
-    return reinterpret_cast<const uint16_t*>(kptr[btab[wave + W * i]]) +
-           (size_t)kvh * kv_head_stride;
+  const int nsteps = (nt + 31) / 32;
+  const int nsw = wave < nsteps ? (nsteps - wave + W - 1) / W : 0;  // this wave's steps
+
+  // Lane l holds the addresses of the wave's l-th block (its steps' blocks in
+  // order; a partition of 4096 tokens has at most 64 per wave); blocks past the
+  // partition repeat its last.
+  uint64_t kp, vp;
+  {
+    const int32_t* btab = block_tables + (size_t)seq * max_blocks + t0 / BS;
+    const int blk = btab[min((wave + W * (lane / NB)) * NB + lane % NB, nb - 1)];
+    const size_t head = (size_t)kvh * kv_head_stride * sizeof(uint16_t);
+    kp = (uint64_t)kptr[blk] + head;
+    vp = (uint64_t)vptr[blk] + head;
+  }
+  auto block_of = [&](uint64_t v, int l) {
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, l);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), l);
+    return ((uint64_t)hi << 32) | lo;
   };
-  auto vbase = [&](int i) {
-    return reinterpret_cast<const uint16_t*>(vptr[btab[wave + W * i]]) +
-           (size_t)kvh * kv_head_stride;
-  };
+  // q . k row c of tile u: token 8 (c / 4) + c % 4 + 4 u of the step
+  const int ktok = 8 * (c >> 2) + (c & 3);
+  const uint32_t koff = (uint32_t)((qd * BS + ktok % BS) * 16);
+  const uint32_t voff = (uint32_t)((c * BS + (8 * qd) % BS) * 2);
+  h8 kreg[SLOTS][2][NK], vreg[SLOTS][ND];
   auto load_k = [&](int slot, int i) {
-    const uint16_t* kb = kbase(i);
-#pragma unroll
-    for (int j = 0; j < SPL; ++j) {
-      if (KTAIL && sg + TPL * j >= SLICES) {
-        kreg[slot][j] = h8{};
-        continue;
-      }
-      kreg[slot][j] = *(const h8*)(kb + ((sg + TPL * j) * BS + tt) * 8);
+    uint64_t base = block_of(kp, i * NB);
+    if (NB == 2) {
+      const uint64_t second = block_of(kp, i * NB + 1);
+      base = c < 8 ? base : second;
     }
+    const unsigned char* kb = reinterpret_cast<const unsigned char*>(base) + koff;
+#pragma unroll
+    for (int j = 0; j < NK; ++j)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        if (SLICES % 4 != 0 && 4 * j + qd >= SLICES) kreg[slot][u][j] = h8{};
+        else kreg[slot][u][j] = *(const h8*)(kb + j * (4 * BS * 16) + u * 64);
+      }
   };
   auto load_v = [&](int slot, int i) {
-    const uint16_t* vb = vbase(i);
+    uint64_t base = block_of(vp, i * NB);
+    if (NB == 2) {
+      const uint64_t second = block_of(vp, i * NB + 1);
+      base = qd < 2 ? base : second;
+    }
+    const unsigned char* vb = reinterpret_cast<const unsigned char*>(base) + voff;
 #pragma unroll
-    for (int j = 0; j < DPL; ++j)
-#pragma unroll
-      for (int u = 0; u < BS / 8; ++u)
-        vreg[slot][j][u] = VTAIL && lane + 64 * j >= HS
-                               ? h8{}
-                               : *(const h8*)(vb + (size_t)(lane + 64 * j) * BS + 8 * u);
+    for (int j = 0; j < ND; ++j) vreg[slot][j] = *(const h8*)(vb + j * (16 * BS * 2));
   };
 #pragma unroll
-  for (int u = 0; u < NPF; ++u)
-    if (u < nbw) {
+  for (int u = 0; u < SLOTS; ++u)
+    if (u < nsw) {
       load_k(u, u);
       load_v(u, u);
     }
-  // The query is staged after the first blocks' key and value loads went
-  // out (each behind its block-table and block-pointer loads), so its own
-  // load overlaps theirs; the barrier that publishes it waits only for the
-  // LDS stores, and the key/value loads stay in flight across it (a
-  // __syncthreads would wait for them).
-  for (int i = tid; i < G * HS; i += (W * 64)) {
-    const int g = i / HS, d = i % HS;
-    qs[i] = scale * (float)as_h(query[(size_t)seq * q_stride + (size_t)(h0 + g) * HS + d]);
+  // the group's queries as B operands: column c is head h0 + c, zero past G
+  h8 qreg[NK];
+  {
+    const uint16_t* qp = query + (size_t)seq * q_stride + (size_t)(h0 + min(c, G - 1)) * HS + 8 * qd;
+#pragma unroll
+    for (int j = 0; j < NK; ++j)
+      qreg[j] = c < G && 4 * j + qd < SLICES ? *(const h8*)(qp + 32 * j) : h8{};
   }
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  const float slope = alibi != nullptr && c < G ? alibi[h0 + c] : 0.f;
 
-  // q . k
-  auto qk = [&](int slot, int i) {
-    const int b = wave + W * i;
-    float dot[GMAX];
+  float m = -FLT_MAX, l = 0.f;  // of head c (l: this lane's tokens)
+  f4 o[ND];
 #pragma unroll
-    for (int g = 0; g < GMAX; ++g) {
-      dot[g] = 0.f;
-      if (g < G) {
+  for (int j = 0; j < ND; ++j) o[j] = f4{0.f, 0.f, 0.f, 0.f};
+  h8 phi, plo;
+  auto softmax = [&](int slot, int i) {
+    f4 s[2] = {f4{0.f, 0.f, 0.f, 0.f}, f4{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-        for (int j = 0; j < SPL; ++j) {
-          if (KTAIL && sg + TPL * j >= SLICES) continue;
-          const float* qv = qs + g * HS + (sg + TPL * j) * 8;
+    for (int j = 0; j < NK; ++j)
 #pragma unroll
-          for (int e = 0; e < 8; ++e) dot[g] = fmaf(qv[e], (float)kreg[slot][j][e], dot[g]);
-        }
-      }
+      for (int u = 0; u < 2; ++u) s[u] = mfma16(kreg[slot][u][j], qreg[j], s[u]);
+    const int t = t0 + (wave + W * i) * 32 + 8 * qd;  // token of element 0
+    float lg[8], mx = -FLT_MAX;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      float v = scale * s[e >> 2][e & 3];
+      if (alibi != nullptr) v += slope * (float)(t + e - ctx + 1);
+      lg[e] = t + e < t1 ? v : -FLT_MAX;
+      mx = fmaxf(mx, lg[e]);
     }
+    mx = fmaxf(mx, __shfl_xor(mx, 16));
+    mx = fmaxf(mx, __shfl_xor(mx, 32));
+    const float mn = fmaxf(m, mx);
+    if (__any(mn != m)) {
+      const float a = exp_of(m - mn);
+      l *= a;
 #pragma unroll
-    for (int g = 0; g < GMAX; ++g) {
-#pragma unroll
-      for (int off = BS; off < 64; off <<= 1) dot[g] += __shfl_xor(dot[g], off);
+      for (int j = 0; j < ND; ++j) o[j] *= a;
     }
-    const int t = t0 + b * BS + tt;
-    if (sg == 0) {
+    m = mn;
 #pragma unroll
-      for (int g = 0; g < GMAX; ++g) {
-        if (g < G) {
-          float l = dot[g];
-          if (alibi != nullptr) l += alibi[h0 + g] * (float)(t - ctx + 1);
-          logit[g * part_tokens + b * BS + tt] = t < t1 ? l : -FLT_MAX;
-        }
-      }
+    for (int e = 0; e < 8; ++e) {
+      const float p = t + e < t1 ? exp_of(lg[e] - mn) : 0.f;
+      l += p;
+      const float ps = p * kPScale;
+      // p > 0 keeps both parts > 0 (at least fp16's smallest), so p times an
+      // infinite value is that infinity
+      const float least = fminf(ps * 0x1p100f, 0x1p-24f);
+      const h2 hi = __builtin_bit_cast(h2, __builtin_amdgcn_cvt_pkrtz(fmaxf(ps, least), 0.f));
+      const h2 lo = __builtin_bit_cast(
+          h2, __builtin_amdgcn_cvt_pkrtz(fmaxf(ps - (float)hi[0], least), 0.f));
+      phi[e] = hi[0];
+      plo[e] = lo[0];
     }
   };
-  for (int i0 = 0; i0 < nbw; i0 += NPF) {
-#pragma unroll
-    for (int u = 0; u < NPF; ++u) {
-      const int i = i0 + u;
-      if (i < nbw) {
-        qk(u, i);
-        if (i + NPF < nbw) load_k(u, i + NPF);
-      }
-    }
-  }
-  __syncthreads();
-
-  // softmax numerators and their sums, per query head
-  float mx[GMAX], sum[GMAX];
-#pragma unroll
-  for (int g = 0; g < GMAX; ++g) {
-    mx[g] = -FLT_MAX;
-    sum[g] = 0.f;
-    if (g < G) {
-      float m = -FLT_MAX;
-      for (int t = tid; t < nt; t += (W * 64)) m = fmaxf(m, logit[g * part_tokens + t]);
-      mx[g] = block_reduce<true, W>(m, scratch);
-      float s = 0.f;
-      for (int t = tid; t < nb * BS; t += (W * 64)) {
-        const float p = t < nt ? __expf(logit[g * part_tokens + t] - mx[g]) : 0.f;
-        logit[g * part_tokens + t] = p;
-        s += p;
-      }
-      sum[g] = block_reduce<false, W>(s, scratch);
-    }
-  }
-  __syncthreads();
-
-  // p . v: lane holds dims lane + 64 j for every query head of the group
-  float acc[GMAX][DPL];
-#pragma unroll
-  for (int g = 0; g < GMAX; ++g)
-#pragma unroll
-    for (int j = 0; j < DPL; ++j) acc[g][j] = 0.f;
   auto pv = [&](int slot, int i) {
-    const int b = wave + W * i;
-    const int valid = min(BS, nt - b * BS);  // tokens of this block in the context
+    const int t = (wave + W * i) * 32;  // within the partition
+    if (t + 32 > nt) {
+      // slots past the context may hold anything: never multiply them
+      const int valid = nt - t - 8 * qd;
 #pragma unroll
-    for (int j = 0; j < DPL; ++j)
+      for (int j = 0; j < ND; ++j)
 #pragma unroll
-      for (int u = 0; u < BS / 8; ++u)
+        for (int e = 0; e < 8; ++e)
+          vreg[slot][j][e] = e < valid ? vreg[slot][j][e] : (_Float16)0.f;
+    }
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int tb = 8 * u + e;
-          // slots past the context may hold anything: never multiply them
-          const float vf = tb < valid ? (float)vreg[slot][j][u][e] : 0.f;
-#pragma unroll
-          for (int g = 0; g < GMAX; ++g)
-            if (g < G) acc[g][j] = fmaf(logit[g * part_tokens + b * BS + tb], vf, acc[g][j]);
-        }
+    for (int j = 0; j < ND; ++j) {
+      o[j] = mfma16(vreg[slot][j], phi, o[j]);
+      o[j] = mfma16(vreg[slot][j], plo, o[j]);
+    }
   };
-  for (int i0 = 0; i0 < nbw; i0 += NPF) {
+  for (int i0 = 0; i0 < nsw; i0 += SLOTS) {
 #pragma unroll
-    for (int u = 0; u < NPF; ++u) {
+    for (int u = 0; u < SLOTS; ++u) {
       const int i = i0 + u;
-      if (i < nbw) {
+      if (i < nsw) {
+        softmax(u, i);
+        if (i + SLOTS < nsw) load_k(u, i + SLOTS);
         pv(u, i);
-        if (i + NPF < nbw) load_v(u, i + NPF);
+        if (i + SLOTS < nsw) load_v(u, i + SLOTS);
       }
     }
   }
+
+  // ---- the waves' outputs, combined in wave order
+  l += __shfl_xor(l, 16);
+  l += __shfl_xor(l, 32);
+  if (c < G) {
 #pragma unroll
-  for (int g = 0; g < GMAX; ++g)
-#pragma unroll
-    for (int j = 0; j < DPL; ++j)
-      if (g < G && (!VTAIL || lane + 64 * j < HS)) red[(wave * GMAX + g) * HS + lane + 64 * j] = acc[g][j];
+    for (int j = 0; j < ND; ++j) *(f4*)(red + (wave * G + c) * HS + j * 16 + 4 * qd) = o[j];
+    if (qd == 0) {
+      ml[(wave * G + c) * 2] = m;
+      ml[(wave * G + c) * 2 + 1] = l;
+    }
+  }
   __syncthreads();
-  for (int i = tid; i < G * HS; i += (W * 64)) {
+  for (int i = tid; i < G * HS; i += W * 64) {
     const int g = i / HS, d = i % HS;
-    float o = 0.f;
+    float gm = ml[g * 2];
 #pragma unroll
-    for (int w = 0; w < W; ++w) o += red[(w * GMAX + g) * HS + d];
-    float s = 0.f, m = 0.f;
+    for (int w = 1; w < W; ++w) gm = fmaxf(gm, ml[(w * G + g) * 2]);
+    float sum = 0.f, acc = 0.f;
 #pragma unroll
-    for (int gg = 0; gg < GMAX; ++gg)
-      if (gg == g) { s = sum[gg]; m = mx[gg]; }
+    for (int w = 0; w < W; ++w) {
+      const float a = exp_of(ml[(w * G + g) * 2] - gm);
+      sum += a * ml[(w * G + g) * 2 + 1];
+      acc += a * red[(w * G + g) * HS + d];
+    }
+    acc *= 1.f / kPScale;
     if (direct) {
-      out[(size_t)seq * o_stride + (size_t)(h0 + g) * HS + d] = h_bits((_Float16)(o / s));
+      out[(size_t)seq * o_stride + (size_t)(h0 + g) * HS + d] = h_bits((_Float16)(acc / sum));
     } else {
       const size_t r = ((size_t)seq * num_heads + h0 + g) * num_parts + part;
-      ws_out[r * HS + d] = o;
+      ws_out[r * HS + d] = acc;
       if (d == 0) {
-        ws_ml[2 * r] = m;
-        ws_ml[2 * r + 1] = s;
+        ws_ml[2 * r] = gm;
+        ws_ml[2 * r + 1] = sum;
       }
     }
   }
@@ -512,30 +728,46 @@ cache_tile_kernel(uint16_t* __restrict__ key, int64_t key_stride, uint16_t* __re
   }
 }
 
-template <int HS, int BS, int GMAX, int W>
+template <int HS, int BS, int W>
 hipError_t launch_pa_w(const PagedAttnArgs& a, const PagedAttnPlan& p, float* ws,
                        hipStream_t stream) {
-  const size_t smem = attn_smem_bytes(HS, GMAX, p.part_tokens, W);
+  const size_t smem = attn_smem_bytes(HS, a.num_heads / a.num_kv_heads, W);
   const dim3 grid((unsigned)(a.num_seqs * a.num_kv_heads), (unsigned)p.num_parts);
   float* ws_ml = p.num_parts > 1 ? ws : nullptr;
   float* ws_out = p.num_parts > 1 ? ws + 2 * (size_t)a.num_seqs * a.num_heads * p.num_parts : nullptr;
-  paged_attention_kernel<HS, BS, GMAX, W><<<grid, W * 64, smem, stream>>>(
+  paged_attention_kernel<HS, BS, W><<<grid, W * 64, smem, stream>>>(
       a.query, a.q_stride, a.out, a.o_stride, a.kptr, a.vptr, a.kv_head_stride, a.num_heads,
       a.num_kv_heads, a.scale, a.block_tables, a.max_blocks, a.context_lens, a.alibi,
       p.part_tokens, p.num_parts, ws_ml, ws_out);
   return hipGetLastError();
 }
 
-template <int HS, int BS, int GMAX>
+template <int HS, int BS, int W>
+hipError_t launch_pa_row(const PagedAttnArgs& a, const PagedAttnPlan& p, float* ws,
+                         hipStream_t stream) {
+  const size_t smem = attn_row_smem_bytes(HS, p.part_tokens, W);
+  const dim3 grid((unsigned)(a.num_seqs * a.num_heads), (unsigned)p.num_parts);
+  float* ws_ml = p.num_parts > 1 ? ws : nullptr;
+  float* ws_out = p.num_parts > 1 ? ws + 2 * (size_t)a.num_seqs * a.num_heads * p.num_parts : nullptr;
+  paged_attention_row_kernel<HS, BS, W><<<grid, W * 64, smem, stream>>>(
+      a.query, a.q_stride, a.out, a.o_stride, a.kptr, a.vptr, a.kv_head_stride, a.num_heads,
+      a.scale, a.block_tables, a.max_blocks, a.context_lens, a.alibi, p.part_tokens, p.num_parts,
+      ws_ml, ws_out);
+  return hipGetLastError();
+}
+
+template <int HS, int BS>
 hipError_t launch_pa(const PagedAttnArgs& a, const PagedAttnPlan& p, float* ws,
                      hipStream_t stream) {
-  hipError_t e;
-  if constexpr (attn_wide_ok(HS, BS, GMAX)) {
-    e = p.waves == 16 ? launch_pa_w<HS, BS, GMAX, 16>(a, p, ws, stream)
-                      : launch_pa_w<HS, BS, GMAX, 4>(a, p, ws, stream);
+  hipError_t e = hipErrorInvalidValue;
+  if (a.num_heads == a.num_kv_heads) {
+    if (p.waves == 4) e = launch_pa_row<HS, BS, 4>(a, p, ws, stream);
+    if constexpr (HS <= 128 && BS == 16)
+      if (p.waves == 16) e = launch_pa_row<HS, BS, 16>(a, p, ws, stream);
   } else {
-    if (p.waves != 4) return hipErrorInvalidValue;
-    e = launch_pa_w<HS, BS, GMAX, 4>(a, p, ws, stream);
+    if (p.waves == 4) e = launch_pa_w<HS, BS, 4>(a, p, ws, stream);
+    if constexpr (HS <= 128)
+      if (p.waves == 8) e = launch_pa_w<HS, BS, 8>(a, p, ws, stream);
   }
   if (e != hipSuccess || p.num_parts == 1) return e;
   float* ws_ml = ws;
@@ -546,20 +778,11 @@ hipError_t launch_pa(const PagedAttnArgs& a, const PagedAttnPlan& p, float* ws,
   return hipGetLastError();
 }
 
-template <int HS, int BS>
-hipError_t launch_pa_g(const PagedAttnArgs& a, const PagedAttnPlan& p, float* ws,
-                       hipStream_t stream) {
-  const int g = a.num_heads / a.num_kv_heads;
-  if (g == 1) return launch_pa<HS, BS, 1>(a, p, ws, stream);
-  if (g <= 4) return launch_pa<HS, BS, 4>(a, p, ws, stream);
-  return launch_pa<HS, BS, 8>(a, p, ws, stream);
-}
-
 template <int HS>
 hipError_t launch_pa_bs(const PagedAttnArgs& a, const PagedAttnPlan& p, float* ws,
                         hipStream_t stream) {
-  if (a.block_size == 16) return launch_pa_g<HS, 16>(a, p, ws, stream);
-  return launch_pa_g<HS, 32>(a, p, ws, stream);
+  if (a.block_size == 16) return launch_pa<HS, 16>(a, p, ws, stream);
+  return launch_pa<HS, 32>(a, p, ws, stream);
 }
 
 // Rotary embedding, rotate-half form, in place on fp16 rows [batch][rows][hd]
@@ -675,23 +898,47 @@ PagedAttnPlan plan_paged_attention(int num_seqs, int num_heads, int num_kv_heads
   PagedAttnPlan p;
   const int blocks = std::max(1, (max_context_len + block_size - 1) / block_size);
   const int pairs = std::max(1, num_seqs * num_kv_heads);
-  // one 16-wave workgroup per (sequence, kv head) over the whole context
-  // where that gives every CU about one workgroup and the context fits one
-  // partition: no combine launch
-  const int g = num_kv_heads > 0 ? num_heads / num_kv_heads : 1;
-  const int gmax = g == 1 ? 1 : g <= 4 ? 4 : 8;
-  if (attn_wide_ok(head_size, block_size, gmax) && 2 * pairs > cus && pairs <= cus &&
-      blocks * block_size <= kAttnWideMaxTokens &&
-      attn_smem_bytes(head_size, gmax, blocks * block_size, 16) <= 64 * 1024) {
-    p.waves = 16;
+  if (num_heads == num_kv_heads) {
+    // one 16-wave workgroup per (sequence, head) over the whole context where
+    // that gives every CU about one workgroup and the context fits one
+    // partition: no combine launch
+    if (head_size <= 128 && block_size == 16 && 2 * pairs > cus && pairs <= cus &&
+        blocks * block_size <= kAttnRowWideTokens) {
+      p.waves = 16;
+      p.part_tokens = blocks * block_size;
+      p.num_parts = 1;
+      return p;
+    }
+    // about four workgroups per CU (eight measured no faster); partitions of
+    // whole blocks, at most 512 tokens
+    const int parts = std::min(std::max(1, (4 * cus + pairs - 1) / pairs), blocks);
+    const int bpp = std::min((blocks + parts - 1) / parts, kAttnRowPartTokens / block_size);
+    p.part_tokens = bpp * block_size;
+    p.num_parts = (blocks + bpp - 1) / bpp;
+    return p;
+  }
+  // One 8-wave workgroup per (sequence, kv head) over the whole context, no
+  // combine launch, where that gives at least half of the CUs one (for
+  // contexts up to 1024 tokens, whose combine launch would count for more, a
+  // third) and none two.  Measured (us, partitioned -> this): 6 x 500 tokens, 32
+  // heads of 128 14.2 -> 11.5; 24 x 3000, 8 kv heads 46.6 -> 42.9; 3 x 800, 40
+  // heads 15.3 -> 12.7.
+  if (head_size <= 128 && pairs <= cus && blocks * block_size <= kAttnWideMaxTokens &&
+      (2 * pairs > cus || (10 * pairs > 3 * cus && blocks * block_size <= 1024))) {
+    p.waves = 8;
     p.part_tokens = blocks * block_size;
     p.num_parts = 1;
     return p;
   }
-  // about four workgroups per CU (eight measured no faster); partitions of
-  // whole blocks, at most 512 tokens
-  int parts = std::max(1, (4 * cus + pairs - 1) / pairs);
-  parts = std::min(parts, blocks);
+  // Otherwise about one 4-wave workgroup per CU, so two on most of the CUs (all
+  // their registers hold); partitions of whole blocks, at least 128 tokens (a
+  // step per wave; 256 for long contexts, whose combine launch reads fewer),
+  // at most 4096.  Measured (us, at least 16 tokens and four workgroups per CU
+  // -> this): 1 x 4000 tokens, 8 kv heads 31.3 -> 12.1; 32 x 1000 28.2 -> 22.8;
+  // 8 x 3000, 16 heads of 256 61.0 -> 54.4.
+  const int least = max_context_len > 2048 ? 256 : 128;
+  int parts = (cus + pairs - 1) / pairs;
+  parts = std::max(1, std::min(parts, (max_context_len + least - 1) / least));
   int bpp = (blocks + parts - 1) / parts;
   bpp = std::min(bpp, kAttnMaxPartTokens / block_size);
   p.part_tokens = bpp * block_size;
