@@ -872,6 +872,15 @@ int dw4_gemm_t_workspace_size(int m, int k, int n, int group_size, size_t* works
   return DW4_OK;
 }
 
+int dw4_gemm_t_packed(int m, int k, int n, int group_size, int* packed) {
+  const int st = check_shape(k, n, group_size);
+  if (st != DW4_OK) return st;
+  if (m < 0 || !packed) return DW4_ERR_INVALID_ARG;
+  *packed = dw4::gemm_t_beats_dense(dw4::plan_gemm_t(std::max(m, 1), k, n, cu_count()), m, k, n,
+                                    group_size);
+  return DW4_OK;
+}
+
 int dw4_gemm_t(int m, int k, int n, int group_size, const uint16_t* g, int64_t ldg,
                const int32_t* packed_qweight, const int32_t* packed_zeros,
                const uint16_t* packed_scales, const int32_t* perm, uint16_t* out, int64_t ldo,

@@ -21,8 +21,12 @@ struct GemmTArgs {
 struct GemmTPlan {
   int ns = 1;   // N-ranges (their fp32 partials are summed in order)
   int spr = 0;  // strips per N-range
+  int mt = 0;   // 16-row tiles per workgroup of the tall form, or 0: up to 64 rows
+  double us = 0;  // modelled time of the tall form
 };
 GemmTPlan plan_gemm_t(int m, int k, int n, int cus);
+// Whether the packed product is expected below dequantisation + a dense product.
+bool gemm_t_beats_dense(const GemmTPlan& p, int m, int k, int n, int gs);
 size_t gemm_t_ws_bytes(const GemmTPlan& p, int m, int k);
 hipError_t launch_gemm_t(const GemmTArgs& a, const GemmTPlan& p, float* part, hipStream_t stream);
 

@@ -94,6 +94,8 @@ SIGNATURES = {
     "dw4_stream_read": (_c.c_int, [_P, _c.c_size_t, _c.c_int, _c.c_int, _c.c_uint32, _P, _P]),
     "dw4_gemm_t": (_c.c_int, [_c.c_int, _c.c_int, _c.c_int, _c.c_int, _P, _c.c_int64, _P, _P, _P,
                               _P, _P, _c.c_int64, _P, _c.c_size_t, _P]),
+    "dw4_gemm_t_packed": (_c.c_int, [_c.c_int, _c.c_int, _c.c_int, _c.c_int,
+                                     _c.POINTER(_c.c_int)]),
     "dw4_gemm_t_workspace_size": (_c.c_int, [_c.c_int, _c.c_int, _c.c_int, _c.c_int,
                                              _c.POINTER(_c.c_size_t)]),
     "dw4_reshape_and_cache": (_c.c_int, [_c.c_int, _c.c_int, _c.c_int, _c.c_int, _P, _c.c_int64,
@@ -206,6 +208,13 @@ def workspace_size(m: int, k: int, n: int, group_size: int, act_order: bool) -> 
     check("dw4_workspace_size", lib.dw4_workspace_size(m, k, n, group_size, int(act_order),
                                                        ctypes.byref(out)))
     return out.value
+
+
+def gemm_t_packed(m: int, k: int, n: int, group_size: int) -> bool:
+    """Whether dw4_gemm_t is expected to beat dequantise + dense product."""
+    out = ctypes.c_int(0)
+    check("dw4_gemm_t_packed", load().dw4_gemm_t_packed(m, k, n, group_size, ctypes.byref(out)))
+    return out.value != 0
 
 
 def gemm_t_workspace_size(m: int, k: int, n: int, group_size: int) -> int:

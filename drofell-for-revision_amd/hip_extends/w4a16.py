@@ -48,9 +48,9 @@ class TuningParams:
     MAX_M: int = 4096
     # Prefill split-K factor; 0 lets the library choose from the tile count.
     PREFILL_SPLIT_K: int = 0
-    # Flattened M up to which the transposed product (PEFT backward) runs the
-    # packed kernel; above it the weight is dequantised and a dense GEMM runs,
-    # as in the reference.
+    # Flattened M up to which the transposed product (PEFT backward) always runs
+    # the packed kernel; above it the library's rule chooses between that and
+    # dequantising and a dense GEMM, as in the reference (0: always the latter).
     TRANSPOSE_MAX_M: int = 128
 
 
@@ -135,6 +135,14 @@ def _output_rows(output: torch.Tensor, m: int, n: int, dtype: torch.dtype) -> to
             and output.stride(0) >= n:
         return output
     raise ValueError("output must be contiguous or a [m, n] view with unit column stride")
+
+
+def _untracked(t: torch.Tensor) -> bool:
+    """Whether t's data alone is the input of a call: no gradient is recorded
+    for it, no vmap or other transform wraps it and it carries no tangent."""
+    return not (t.requires_grad and torch.is_grad_enabled()) \
+        and not torch._C._functorch.is_functorch_wrapped_tensor(t) \
+        and torch.autograd.forward_ad.unpack_dual(t).tangent is None
 
 
 def _aligned_rows(x2: torch.Tensor) -> torch.Tensor:
@@ -421,8 +429,12 @@ class Q4MatrixV2(object):
         return self.reconstructed_weight_float16 if dtype == torch.float16 else \
             self.reconstructed_weight_bfloat16
 
-    def _transpose_native(self, x: torch.Tensor, output: Optional[torch.Tensor]) -> torch.Tensor:
-        """fp16 ``x @ W.T`` through the packed transposed kernel."""
+    def _transpose_native(self, x: torch.Tensor, output: Optional[torch.Tensor],
+                          own_workspace: bool = False) -> torch.Tensor:
+        """fp16 ``x @ W.T`` through the packed transposed kernel; the fp32
+        planes in the shared workspace or, with ``own_workspace``, in one of
+        this call (the size grows with M, and a captured graph or another
+        stream may hold the shared one)."""
         if x.device != self.device:
             raise ValueError(f"input on {x.device}, weights on {self.device}")
         if x.dtype != torch.float16:
@@ -433,7 +445,8 @@ class Q4MatrixV2(object):
         out2 = torch.empty((m, self.height), dtype=torch.float16, device=self.device) \
             if output is None else _output_rows(output, m, self.height, torch.float16)
         nbytes = _lib.gemm_t_workspace_size(m, self.height, self.width, self.group_size)
-        ws = self.cache.transpose_workspace(nbytes)
+        ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=self.device) \
+            if own_workspace else self.cache.transpose_workspace(nbytes)
         _lib.call("dw4_gemm_t", m, self.height, self.width, self.group_size,
                   g2.data_ptr(), g2.stride(0), self.qweight.data_ptr(), self.qzeros.data_ptr(),
                   self.scales.data_ptr(), _ptr(self.perm) if self.use_act else None,
@@ -502,6 +515,16 @@ class Q4MatrixV2(object):
         if dtype in (None, torch.bfloat16):
             self.reconstructed_weight_bfloat16 = None
 
+    def _packed_rows(self, m: int, dtype: torch.dtype) -> bool:
+        """Whether the transposed product of m rows runs on the packed words."""
+        limit = self.tuning_params.TRANSPOSE_MAX_M
+        return dtype == torch.float16 and m > 0 and limit > 0 and (
+            m <= limit or _lib.gemm_t_packed(m, self.height, self.width, self.group_size))
+
+    def packed_transpose(self, x: torch.Tensor) -> bool:
+        """Whether the gradient of forward input x [..., K] takes the packed words."""
+        return x.device == self.device and self._packed_rows(x.numel() // self.height, x.dtype)
+
     def transpose_matmul(self, x: torch.Tensor, output: Optional[torch.Tensor] = None,
                          temp_weight: Optional[torch.Tensor] = None,
                          skip_reconstruct: bool = False) -> torch.Tensor:
@@ -513,7 +536,10 @@ class Q4MatrixV2(object):
         already filled ``temp_weight``), the product is the dense one over
         that weight.  Otherwise fp16 x up to ``TuningParams.TRANSPOSE_MAX_M``
         rows runs the packed kernel (``dw4_gemm_t``), which reads the int4
-        words directly; above it, and for bf16 x, the weight is dequantised
+        words directly, and so does fp16 x above it where the library expects
+        that to be faster, unless the limit is 0, ``temp_weight`` or
+        ``output`` is given (the caller may read the weight; x may overlap
+        the output) or a transform follows x.  Else the weight is dequantised
         bit-exactly (fp16, or bf16 of the fp16 value) into ``temp_weight`` or
         the shared buffer and a library GEMM runs, as in the reference.
         """
@@ -526,6 +552,9 @@ class Q4MatrixV2(object):
         if w is None and not skip_reconstruct and dtype == torch.float16 \
                 and 0 < m <= self.tuning_params.TRANSPOSE_MAX_M:
             return self._transpose_native(x, output)
+        if w is None and not skip_reconstruct and temp_weight is None and output is None \
+                and x.device == self.device and _untracked(x) and self._packed_rows(m, dtype):
+            return self._transpose_native(x, None, own_workspace=True)
         if w is None:
             if skip_reconstruct:
                 if temp_weight is None:
@@ -548,7 +577,10 @@ class Q4LinearFunction(Function):
 
     As ``ExllamaQ4LinearFunction`` (``exllama.py:649-696``): with
     ``cache_weight`` the dequantised weight of the input's dtype is kept for
-    the backward (unless the matrix already holds a reconstructed one);
+    the backward, unless the matrix already holds a reconstructed one or the
+    backward runs on the packed words (fp16 rows up to the library's rule,
+    where writing the dense weight costs more than it saves: 128 rows on
+    4096 x 11008 74 us to write and use, against 29 packed);
     the forward of fp16 input still runs the W4A16 kernel, bf16 input the
     dense product over the kept weight.
     """
@@ -558,7 +590,8 @@ class Q4LinearFunction(Function):
                 bias: Optional[torch.Tensor], cache_weight: bool) -> torch.Tensor:
         ctx.weight_q4 = weight_q4
         cached = None
-        if cache_weight and weight_q4._reconstructed(input.dtype) is None:
+        ctx.own_weight = cache_weight and weight_q4._reconstructed(input.dtype) is None
+        if ctx.own_weight and not weight_q4.packed_transpose(input):
             cached = weight_q4._dense_weight(
                 torch.empty(weight_q4.height * weight_q4.width, dtype=input.dtype,
                             device=weight_q4.device), input.dtype)
@@ -578,6 +611,13 @@ class Q4LinearFunction(Function):
             if ctx.has_cached:
                 grad_input = ctx.weight_q4.transpose_matmul(
                     grad_output, None, ctx.saved_tensors[0], skip_reconstruct=True)
+            elif ctx.own_weight and not _untracked(grad_output):
+                # recorded or transformed: the dense product over a weight of
+                # its own, which a later backward of this one may read
+                q4 = ctx.weight_q4
+                own = q4._dense_weight(torch.empty(q4.height * q4.width, dtype=grad_output.dtype,
+                                                   device=q4.device), grad_output.dtype)
+                grad_input = q4.transpose_matmul(grad_output, None, own, skip_reconstruct=True)
             else:
                 grad_input = ctx.weight_q4.transpose_matmul(grad_output)
         return grad_input, None, None, None

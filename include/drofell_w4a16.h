@@ -284,6 +284,9 @@ int dw4_gemm_t(int m, int k, int n, int group_size, const uint16_t* g, int64_t l
                const uint16_t* packed_scales, const int32_t* perm, uint16_t* out, int64_t ldo,
                void* workspace, size_t workspace_bytes, void* stream);
 int dw4_gemm_t_workspace_size(int m, int k, int n, int group_size, size_t* workspace_bytes);
+/* *packed = 1 where dw4_gemm_t is expected to be faster than dequantising and
+ * a dense product (above 64 rows a fitted time decides), else 0. */
+int dw4_gemm_t_packed(int m, int k, int n, int group_size, int* packed);
 
 /* ---------------------------------------------------------------------------
  * Decoder-stage calls: several projections of one layer per launch.

@@ -142,3 +142,79 @@ def test_transpose_status(hip_device):
         assert lib.dw4_gemm_t(4, 1024, 512, 32, g.data_ptr(), 512, *args, None, 0, None) == \
             _lib.DW4_ERR_WORKSPACE
     assert lib.dw4_gemm_t(0, 1024, 512, 32, None, 512, *args, None, 0, None) == _lib.DW4_OK
+
+
+# Tiles of 48 and 64 rows with their remainders, an odd number of strips (the
+# last in a pair of its own), one chunk row, N-ranges, groups of 32 to K.  The
+# weight is exact in both, so the bound is the fp16 rounding of the result
+# (2^-11) plus fp32 sums of n products (n 2^-24 of the sum of magnitudes).
+@pytest.mark.parametrize("k,n,group,act", [
+    (128, 16, 32, False), (128, 48, 128, False), (256, 272, 64, True), (1152, 1056, 128, True),
+    (512, 4112, 512, False), (4096, 4096, 128, False)])
+def test_tall_rows_edges(hip_device, k, n, group, act):
+    lay, w = _layer(k, n, group, 8100 + k + n, act)
+    q4 = _matrix(lay, hip_device)
+    wd = w.astype(np.float64)
+    for m in (65, 96, 97, 128, 129, 385):
+        say(f"tall gemm_t {k}x{n} g={group} act={act} M={m}")
+        g = make_x(m, n, seed=8200 + m)
+        gd = g.numpy().astype(np.float64)
+        out = _gemm_t(q4, g.to(hip_device)).double().cpu().numpy()
+        bound = 2.0 ** -11 * np.abs(gd @ wd.T) + n * 2.0 ** -24 * (np.abs(gd) @ np.abs(wd).T) + 2.0 ** -24
+        assert np.all(np.abs(out - gd @ wd.T) <= bound), (m, k, n)
+
+
+def test_tall_overflowing_weight_stays_at_its_output(hip_device):
+    # s (q - z) beyond fp16 in one group of one column: infinite weights at
+    # some of its rows k only, and the other outputs as the dense product has them
+    lay, _ = _layer(256, 64, 128, 8300, False)
+    scales = lay.scales.clone()
+    scales[1, 5] = 30000.0
+    cache = CacheV2(hip_device)
+    q4 = Q4MatrixV2(*(t.to(hip_device) for t in (lay.qweight, lay.qzeros, scales)), 256, 64, None, False,
+                    TuningParams(MAX_M=256, TRANSPOSE_MAX_M=128), cache)
+    cache.init_cache()
+    g = (make_x(200, 64, seed=8301) * 0.01).to(hip_device)
+    w = q4.get_float16_weights_matrix_v2()
+    finite = torch.isfinite(w).all(dim=1)
+    assert finite.any() and not finite.all()
+    say("tall gemm_t with overflowing weights")
+    out = _gemm_t(q4, g).float()
+    ref = g.float() @ w.float().t().contiguous()
+    assert torch.isfinite(out[:, finite]).all()
+    assert torch.equal(out[:, ~finite], ref[:, ~finite])
+
+
+def test_transpose_above_limit_keeps_dense_semantics(hip_device):
+    lay, w = _layer(1152, 1056, 128, 8400, True)
+    q4 = _matrix(lay, hip_device)
+    q4.tuning_params = TuningParams(TRANSPOSE_MAX_M=64)
+    assert _lib.gemm_t_packed(200, 1152, 1056, 128)
+    g = make_x(200, 1056, seed=8401).to(hip_device)
+    say("packed above the limit, then the calls that keep the dense product")
+    _check(q4.transpose_matmul(g), g.cpu(), w, "packed")
+    buf = torch.zeros(1152 * 1056, dtype=torch.float16, device=hip_device)
+    q4.transpose_matmul(g, None, buf)
+    assert torch.equal(buf.view(1152, 1056), q4.get_float16_weights_matrix_v2())
+    tracked = g.clone().requires_grad_(True)
+    assert q4.transpose_matmul(tracked).requires_grad
+    out = torch.func.vmap(q4.transpose_matmul)(g.view(2, 100, 1056))
+    _check(out.view(200, 1152), g.cpu(), w, "vmap")
+
+
+@pytest.mark.parametrize("m", [1, 384, 3000])
+def test_backward_with_kept_weight(hip_device, m):
+    lay, w = _layer(1152, 1056, 128, 8500, True)
+    q4 = _matrix(lay, hip_device)
+    q4.tuning_params = TuningParams(MAX_M=256)
+    x = make_x(m, 1152, seed=8501).to(hip_device).requires_grad_(True)
+    dy = make_x(m, 1056, seed=8502).to(hip_device)
+    say(f"gradient with the weight kept, M={m}: first order, and recorded")
+    y = Q4LinearFunction.apply(x, q4, None, True)
+    dx, = torch.autograd.grad(y, x, dy, retain_graph=True)
+    _check(dx, dy.cpu(), w, "gradient")
+    tracked = dy.clone().requires_grad_(True)
+    dx2, = torch.autograd.grad(y, x, tracked, create_graph=True)
+    q4.cache.temp_weight.zero_()
+    ddy, = torch.autograd.grad(dx2, tracked, x.detach())
+    _check(ddy, x.detach().cpu(), w.T, "second order")
