@@ -359,8 +359,10 @@ class Q4MatrixV2(object):
           packed words, the exact s * (q - z) applied per group in fp32, bf16
           output, one launch), between the two the HIP prefill kernels
           (``dw4_gemm_bf16_prefill``: the weight rounded once to bf16 in the
-          kernel), within rounding of the dense product.  The activations
-          keep bf16's range either way.
+          kernel), within rounding of the dense product, unless
+          ``temp_weight`` is given (it is filled) or a gradient or transform
+          follows x or the bias.  The activations keep bf16's range either
+          way.
 
         ``output`` (x's dtype, ``M * N`` elements, contiguous or a row-strided
         [M, N] view) receives the product; anything else raises.  ``bias``
@@ -380,7 +382,9 @@ class Q4MatrixV2(object):
             bias = bias.to(dtype).contiguous()
         dense = self._reconstructed(dtype)
         if dtype == torch.bfloat16 and dense is None and not must_blas \
-                and 0 < m <= _lib.BF16_PREFILL_MAX_M:
+                and (0 < m <= _lib.BF16_MAX_M or (
+                    0 < m <= _lib.BF16_PREFILL_MAX_M and temp_weight is None and _untracked(x)
+                    and (bias is None or _untracked(bias)))):
             fn = "dw4_gemm_bf16" if m <= _lib.BF16_MAX_M else "dw4_gemm_bf16_prefill"
             x2 = _aligned_rows(x.reshape(m, self.height))
             y2 = torch.empty((m, self.width), dtype=torch.bfloat16, device=self.device) \

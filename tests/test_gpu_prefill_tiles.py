@@ -168,3 +168,22 @@ def test_wide_row_stride_keeps_the_64_bit_kernel(hip_device):
     y = q4.matmul(xs, path=_lib.DW4_PATH_PREFILL)
     torch.cuda.synchronize()
     _check(y, x, w, None, "wide stride")
+
+
+def test_bf16_rows_keep_dense_semantics(hip_device):
+    # above the decode rows: a given weight buffer is filled, and a recorded
+    # input gets its gradient (dy W^T; bf16 operands, so 2^-8 of each product)
+    lay = make_layer(512, 256, 128, seed=91).to(hip_device)
+    cache = CacheV2(hip_device)
+    q4 = Q4MatrixV2(lay.qweight, lay.qzeros, lay.scales, 512, 256, None, False, TuningParams(MAX_M=256), cache)
+    cache.init_cache()
+    w = q4.get_bfloat16_weights_matrix_v2().float()
+    x = torch.randn(100, 512, device=hip_device).to(torch.bfloat16)
+    buf = torch.zeros(512 * 256, dtype=torch.float16, device=hip_device)
+    say("bf16 100 rows with a weight buffer, then recorded")
+    q4.matmul(x, temp_weight=buf)
+    assert torch.equal(buf.view(torch.bfloat16).view(512, 256).float(), w)
+    tracked = x.clone().requires_grad_(True)
+    dx, = torch.autograd.grad(q4.matmul(tracked).float().sum(), tracked)
+    ref = w.sum(dim=1).expand(100, 512)
+    assert ((dx.float() - ref).abs() <= 2.0 ** -8 * w.abs().sum(dim=1)).all()
