@@ -125,15 +125,7 @@ __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
 }
 
 // A column's group constants for the B operands of the prefill kernels.
-// fp16: the weight is fp16(s (q - z)) from the exact integer q - z.
-// bf16: the weight is bf16(s (q - z)), rounded once: with the nibbles OR-ed
-// into fp16 1024.0 (values 1024 + q and 1024 + 16 q), s (1024 + q) - s (1024 +
-// z) is one mixed-precision FMA whose product, addend and result are exact in
-// fp32 (s has 11 significant bits, 1024 + q at most 11, s (q - z) at most 16).
-template <bool BF>
-struct ColGroup;
-template <>
-struct ColGroup<false> {
+struct ColGroup {
   h2 nz1024, nz64;
   _Float16 s;
   __device__ __forceinline__ void set(uint32_t sword, int hsh, uint32_t zword, int zsh) {
@@ -141,31 +133,21 @@ struct ColGroup<false> {
     s = as_h((uint16_t)(sword >> hsh));
   }
 };
-template <>
-struct ColGroup<true> {
-  float s, c1024, s16, c64;
-  __device__ __forceinline__ void set(uint32_t sword, int hsh, uint32_t zword, int zsh) {
-    s = (float)as_h((uint16_t)(sword >> hsh));
-    const float z = (float)(((zword >> zsh) & 15u) + 1u);
-    c1024 = -s * (1024.f + z);
-    s16 = s * 0.0625f;
-    c64 = -s * (64.f + z);
-  }
-};
 
-// The B operand of 8 rows of one packed word.
-__device__ __forceinline__ h8 weight8(uint32_t w, const ColGroup<false>& g, uint32_t magic) {
-  return centered8(w, g.nz1024, g.nz64, magic) * h8{g.s, g.s, g.s, g.s, g.s, g.s, g.s, g.s};
-}
-__device__ __forceinline__ h8 weight8(uint32_t w, const ColGroup<true>& g, uint32_t magic) {
-  const uint32_t w8 = w >> 8;
-  const h2 p0 = as_h2(and_or(w, 0x000F000Fu, magic)), p1 = as_h2(and_or(w, 0x00F000F0u, magic));
-  const h2 p2 = as_h2(and_or(w8, 0x000F000Fu, magic)), p3 = as_h2(and_or(w8, 0x00F000F0u, magic));
-  return __builtin_bit_cast(
-      h8, u4{pack_bf16(fmaf((float)p0[0], g.s, g.c1024), fmaf((float)p0[1], g.s, g.c1024)),
-             pack_bf16(fmaf((float)p1[0], g.s16, g.c64), fmaf((float)p1[1], g.s16, g.c64)),
-             pack_bf16(fmaf((float)p2[0], g.s, g.c1024), fmaf((float)p2[1], g.s, g.c1024)),
-             pack_bf16(fmaf((float)p3[0], g.s16, g.c64), fmaf((float)p3[1], g.s16, g.c64))});
+// The B operand of 8 rows of one packed word: fp16(s (q - z)) from the exact
+// integer q - z, and for bf16 activations (BF) that value rounded again to
+// bf16.  Both roundings, as in the dequantised bf16 weight: bf16(s (q - z))
+// rounded once would save 8 of 25 vector instructions, but differs from it in
+// one value of thirty, gives NaN where an infinite scale gives infinities,
+// and finite weights where the dequantised one overflows fp16.
+template <bool BF>
+__device__ __forceinline__ h8 weight8(uint32_t w, const ColGroup& g, uint32_t magic) {
+  const h8 v = centered8(w, g.nz1024, g.nz64, magic) * h8{g.s, g.s, g.s, g.s, g.s, g.s, g.s, g.s};
+  if constexpr (BF)
+    return __builtin_bit_cast(h8, u4{pack_bf16((float)v[0], (float)v[1]), pack_bf16((float)v[2], (float)v[3]),
+                                     pack_bf16((float)v[4], (float)v[5]), pack_bf16((float)v[6], (float)v[7])});
+  else
+    return v;
 }
 
 typedef float f16v __attribute__((ext_vector_type(16)));

@@ -157,7 +157,7 @@ kslice_kernel(const _Float16* __restrict__ x, int64_t ldx, int M, const P2Items 
     for (int a = 0; a < AI; ++a) *(h8*)(xw + a * 1024) = ab[h][a];
   };
   auto compute = [&](int h) {
-    ColGroup<BF> col[P][GH];
+    ColGroup col[P][GH];
 #pragma unroll
     for (int p = 0; p < P; ++p)
 #pragma unroll
@@ -174,7 +174,7 @@ kslice_kernel(const _Float16* __restrict__ x, int64_t ldx, int M, const P2Items 
         if ((t & 1) == 0)
           strip_pair_to_b32(t ? qb[h][2 * p].y : qb[h][2 * p].x,
                             t ? qb[h][2 * p + 1].y : qb[h][2 * p + 1].x, ev[p], od[p]);
-        const h8 bop = weight8((t & 1) ? od[p] : ev[p], col[p][gl], magic);
+        const h8 bop = weight8<BF>((t & 1) ? od[p] : ev[p], col[p][gl], magic);
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) acc[mt][p] = mfma32_of<BF>(af[mt], bop, acc[mt][p]);
       }

@@ -35,8 +35,8 @@
 //   * dequantisation as everywhere in this library: the exact fp16 weight
 //     fp16_rne(s * (q - z)) from the 0x6400 identity, so the product equals
 //     "dequantise, then an fp32-accumulated matmul"; bf16 activations take
-//     bf16_rne(s * (q - z)), one mixed-precision FMA per value and one packed
-//     conversion per pair (17 instead of 13 vector instructions per fragment);
+//     that fp16 value rounded to bf16, the dequantised bf16 weight (two
+//     conversions per value more, 25 vector instructions per fragment);
 //   * the 96-row tile is for the row counts between the others: M=384 on 4096
 //     x 11008 takes 172 workgroups of it in one round, 49.0 us, against 129
 //     half-filling ones of 128 rows, 59.0, or 258 of 64 rows, two rounds;
@@ -277,7 +277,7 @@ prefill2_kernel(const _Float16* __restrict__ x, int64_t ldx, int M, const P2Item
         qw[si][T::kWords - 1] = v.y;
       }
     }
-    ColGroup<BF> col[kPairs][T::kGroups];
+    ColGroup col[kPairs][T::kGroups];
 #pragma unroll
     for (int p = 0; p < kPairs; ++p)
 #pragma unroll
@@ -294,7 +294,7 @@ prefill2_kernel(const _Float16* __restrict__ x, int64_t ldx, int M, const P2Item
       for (int p = 0; p < kPairs; ++p) {
         if ((tt & 1) == 0)
           strip_pair_to_b32(qw[2 * p][tt >> 1], qw[2 * p + 1][tt >> 1], ev[p], od[p]);
-        bop[p] = weight8((tt & 1) ? od[p] : ev[p], col[p][gl], magic);
+        bop[p] = weight8<BF>((tt & 1) ? od[p] : ev[p], col[p][gl], magic);
       }
     };
     auto read_a = [&](int tt, h8 (&af)[kMT]) {

@@ -132,12 +132,6 @@ SIGNATURES = {
 }
 ABI_VERSION = 11
 BF16_MAX_M = 64  # DW4_BF16_MAX_M
-# Rows up to which bf16 x runs on the packed words (prefill kernels) rather
-# than over a dequantised weight (us, packed against dequantise + library GEMM):
-# M=65 4096^2 14.0 / 37.6, M=256 11008x4096 38.4 / 90.2, M=700 4096x11008 90.0 /
-# 110.6, M=1024 5120x13824 153 / 159, M=1536 235 / 237 there and 152 / 166 at
-# 11008x4096; at M=2048 315 / 284, at M=3072 the dense route wins on every shape.
-BF16_PREFILL_MAX_M = 1536
 
 _lock = threading.Lock()
 _lib: Optional[ctypes.CDLL] = None
@@ -208,6 +202,24 @@ def workspace_size(m: int, k: int, n: int, group_size: int, act_order: bool) -> 
     check("dw4_workspace_size", lib.dw4_workspace_size(m, k, n, group_size, int(act_order),
                                                        ctypes.byref(out)))
     return out.value
+
+
+def bf16_prefill_max_m(k: int, n: int, act_order: bool) -> int:
+    """Rows up to which bf16 x runs on the packed words (prefill kernels)
+    rather than over a dequantised weight.  Measured with the matrices in
+    cache, which favours the dense route (us, packed against dequantise +
+    library GEMM):
+    * N <= K: 700 rows on 4096^2 49.6 / 49.1 (out of cache 49.3 / 58.7), 1536
+      on 11008x4096 147 / 162, on 13824x5120 219 / 241, on 5120^2 86 / 92;
+    * N > K: 640 rows on 4096x22016 130 / 167, 700 on 4096x11008 98.1 / 111,
+      on 5120x13824 133 / 136; 900 there 159 / 155, 1280 on 4096x11008
+      131 / 121;
+    * act-order, which gathers x first: 640 rows on 4096^2 45.2 / 47.5, on
+      4096x12288 76.4 / 93.0, on 5120x13824 136 / 131; 704 rows on 4096^2
+      52.2 / 47.3, on 4096x12288 113 / 101."""
+    if act_order:
+        return 640
+    return 704 if n > k else 1536
 
 
 def gemm_t_packed(m: int, k: int, n: int, group_size: int) -> bool:

@@ -350,7 +350,7 @@ class Q4MatrixV2(object):
           library GEMM); otherwise the HIP W4A16 kernel (decode kernel for
           small M, MFMA prefill kernel above);
         * bf16 x: with a reconstructed bf16 weight, ``must_blas`` or more
-          than ``BF16_PREFILL_MAX_M`` rows, the dense bf16 product (fp32
+          than ``_lib.bf16_prefill_max_m`` rows, the dense bf16 product (fp32
           accumulation) over the bf16 weight bf16(fp16(s * (q - z))), the
           reconstructed one or one dequantised into ``temp_weight`` / the
           shared buffer, as the reference's ``q4_matmul_blas_v2`` with
@@ -358,10 +358,10 @@ class Q4MatrixV2(object):
           kernel's bf16 mode (``dw4_gemm_bf16``: bf16 matrix cores over the
           packed words, the exact s * (q - z) applied per group in fp32, bf16
           output, one launch), between the two the HIP prefill kernels
-          (``dw4_gemm_bf16_prefill``: the weight rounded once to bf16 in the
-          kernel), within rounding of the dense product, unless
-          ``temp_weight`` is given (it is filled) or a gradient or transform
-          follows x or the bias.  The activations keep bf16's range either
+          (``dw4_gemm_bf16_prefill``: the dense product's weight
+          bf16(fp16(s * (q - z))) formed in the kernel, so only the order of
+          the fp32 sums differs), unless ``temp_weight`` is given (it is
+          filled) or a gradient or transform follows x or the bias.  The activations keep bf16's range either
           way.
 
         ``output`` (x's dtype, ``M * N`` elements, contiguous or a row-strided
@@ -383,7 +383,8 @@ class Q4MatrixV2(object):
         dense = self._reconstructed(dtype)
         if dtype == torch.bfloat16 and dense is None and not must_blas \
                 and (0 < m <= _lib.BF16_MAX_M or (
-                    0 < m <= _lib.BF16_PREFILL_MAX_M and temp_weight is None and _untracked(x)
+                    0 < m <= _lib.bf16_prefill_max_m(self.height, self.width, self.use_act)
+                    and temp_weight is None and _untracked(x)
                     and (bias is None or _untracked(bias)))):
             fn = "dw4_gemm_bf16" if m <= _lib.BF16_MAX_M else "dw4_gemm_bf16_prefill"
             x2 = _aligned_rows(x.reshape(m, self.height))

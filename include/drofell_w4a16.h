@@ -192,10 +192,11 @@ int dw4_gemm_bf16(int m, int k, int n, int group_size,
                   const uint16_t* bias, uint16_t* y, int64_t ldy,
                   void* workspace, size_t workspace_bytes, void* stream);
 
-/* Device: the same product for any m >= 1 on the prefill kernels (bf16 matrix
- * cores, the packed words dequantised in the kernel to bf16(s (q - z)), rounded
- * once; fp32 accumulation).  Buffers, alignment, bias and output as in
- * dw4_gemm_bf16.  A K split uses the workspace's planes where they fit.
+/* Device: the product of bf16 x for any m >= 1 on the prefill kernels (bf16
+ * matrix cores, fp32 accumulation, the packed words dequantised in the kernel
+ * to bf16(fp16(s (q - z))), the weight dw4_dequant_bf16 writes).  Buffers,
+ * alignment, bias and output as in dw4_gemm_bf16.  A K split uses the
+ * workspace's planes where they fit.
  * Act-order calls need room for the gathered rows (dw4_workspace_size(m, ...,
  * act_order = 1) bytes, zero-filled once) and return DW4_ERR_WORKSPACE without;
  * row strides of x beyond 2^22 elements return DW4_ERR_UNSUPPORTED (x without

@@ -187,3 +187,45 @@ def test_bf16_rows_keep_dense_semantics(hip_device):
     dx, = torch.autograd.grad(q4.matmul(tracked).float().sum(), tracked)
     ref = w.sum(dim=1).expand(100, 512)
     assert ((dx.float() - ref).abs() <= 2.0 ** -8 * w.abs().sum(dim=1)).all()
+
+
+@pytest.mark.parametrize("m,k,n,g,act", [(100, 512, 400, 128, True), (300, 384, 4112, 64, False),
+                                         (700, 512, 1040, 32, False)])
+def test_bf16_prefill_takes_the_dequantised_weight(hip_device, m, k, n, g, act):
+    """The packed bf16 product is over the very weight of the dense route,
+    bf16(fp16(s (q - z))): against its float64 product only half an ulp of
+    the output and the fp32 sums are left (K terms of random sign, rounded at
+    2^-24 of a partial sum each; twice that).  A weight rounded once, an ulp
+    off in one value of thirty, moves one output in fifteen past this."""
+    q4, _ = _build(k, n, g, act, hip_device, m)
+    w = q4.get_bfloat16_weights_matrix_v2().double().cpu().numpy()
+    x = _x(m, k, torch.bfloat16, m + 1)
+    say(f"bf16 prefill over the dequantised weight {k}x{n} g={g} act={act} M={m}")
+    y = q4.matmul(x.to(hip_device)).double().cpu().numpy()
+    xd = x.double().numpy()
+    ref = xd @ w
+    half_ulp = 2.0 ** (np.floor(np.log2(np.maximum(np.abs(ref), np.abs(y)))) - 8)
+    sums = 2.0 ** -23 * k ** 0.5 * np.sqrt((xd ** 2) @ (w ** 2))
+    bad = np.abs(y - ref) > half_ulp + sums
+    assert not bad.any(), f"{bad.mean():.4f} of the outputs"
+
+
+@pytest.mark.parametrize("scale", [float("inf"), 30000.0])
+def test_bf16_prefill_overflowing_scales(hip_device, scale):
+    """An infinite scale, and one whose weights overflow fp16: infinities and
+    NaN where the dense product over the dequantised weight has them."""
+    lay = make_layer(256, 80, 128, seed=93, symmetric=True)
+    scales = lay.scales.clone()
+    scales[1, 5] = scale
+    qweight = lay.qweight | -0x66666667  # 0x99999999: codes above the zero of 8, weights > 0
+    cache = CacheV2(hip_device)
+    q4 = Q4MatrixV2(*(t.to(hip_device) for t in (qweight, lay.qzeros, scales)), 256, 80, None, False,
+                    TuningParams(MAX_M=128), cache)
+    cache.init_cache()
+    say(f"bf16 prefill with a scale of {scale}")
+    x = _x(100, 256, torch.bfloat16, 5).to(hip_device)
+    x[::2] = x[::2].abs()  # infinite in every other row, inf - inf in the rest
+    y, ref = q4.matmul(x).float(), q4.matmul(x, must_blas=True).float()
+    assert torch.isposinf(ref[::2, 5]).all() and torch.isnan(ref[1::2, 5]).all()
+    assert torch.equal(torch.isnan(y), torch.isnan(ref))
+    assert torch.equal(torch.isposinf(y), torch.isposinf(ref))
