@@ -114,14 +114,12 @@ class DenseRoutePlan:
 
 class MarlinDenseCache:
     """The shared, stream-ordered dense-route buffers of one decoder group
-    (sized by :class:`DenseRoutePlan`), plus the transposed product's
-    partial planes, grown on demand outside graph capture."""
+    (sized by :class:`DenseRoutePlan`)."""
 
     def __init__(self, device: torch.device) -> None:
         self.device = torch.device(device)
         self.plan = DenseRoutePlan()
         self._buffers: Optional[tuple] = None
-        self._t_workspace: Optional[torch.Tensor] = None
 
     @property
     def temp_weight_elements(self) -> int:
@@ -158,13 +156,6 @@ class MarlinDenseCache:
     @property
     def workspace(self) -> torch.Tensor:
         return self._allocated()[1]
-
-    def transpose_workspace(self, nbytes: int) -> torch.Tensor:
-        t = self._t_workspace
-        if t is None or t.numel() < nbytes:
-            t = self._t_workspace = torch.empty(max(nbytes, 16), dtype=torch.uint8,
-                                                device=self.device)
-        return t
 
 
 def make_marlin_workspace(device: torch.device) -> torch.Tensor:
@@ -355,7 +346,9 @@ class MarlinQ4Matrix:
             out = torch.empty((m, self.in_features), dtype=torch.float16, device=x.device)
             nbytes = _lib.gemm_t_workspace_size(m, self.in_features, self.out_features,
                                                 self.group_size)
-            ws = self.cache.transpose_workspace(nbytes)
+            # planes of this call alone: a shared buffer would be written by
+            # several streams and freed under a captured call when it grows
+            ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=x.device)
             _lib.call("dw4_gemm_t", m, self.in_features, self.out_features, self.group_size,
                       g2.data_ptr(), g2.stride(0), self.qweight.data_ptr(),
                       self.qzeros.data_ptr(), self.scales.data_ptr(), _ptr(self._perm),

@@ -69,7 +69,6 @@ class CacheV2(object):
         self.temp_weight_size: int = 0
         self._workspace: Optional[torch.Tensor] = None
         self._temp_weight: Optional[torch.Tensor] = None
-        self._t_workspace: Optional[torch.Tensor] = None
         self.cache_created = False
 
     def update_workspace_size(self, nbytes: int) -> None:
@@ -95,13 +94,6 @@ class CacheV2(object):
         if not self.cache_created or self._workspace is None:
             raise RuntimeError("CacheV2.init_cache() must run before the first matmul")
         return self._workspace
-
-    def transpose_workspace(self, nbytes: int) -> torch.Tensor:
-        """fp32 partial planes of the transposed product, grown on demand
-        (the backward runs outside graph capture); no zero-fill needed."""
-        if self._t_workspace is None or self._t_workspace.numel() < nbytes:
-            self._t_workspace = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=self.device)
-        return self._t_workspace
 
     @property
     def temp_weight(self) -> torch.Tensor:
@@ -434,28 +426,34 @@ class Q4MatrixV2(object):
         return self.reconstructed_weight_float16 if dtype == torch.float16 else \
             self.reconstructed_weight_bfloat16
 
+    def _words(self) -> Tuple[torch.Tensor, ...]:
+        """The packed tensors a product reads."""
+        return self.qweight, self.qzeros, self.scales, self.perm
+
     def _transpose_native(self, x: torch.Tensor, output: Optional[torch.Tensor],
-                          own_workspace: bool = False) -> torch.Tensor:
-        """fp16 ``x @ W.T`` through the packed transposed kernel; the fp32
-        planes in the shared workspace or, with ``own_workspace``, in one of
-        this call (the size grows with M, and a captured graph or another
-        stream may hold the shared one)."""
-        if x.device != self.device:
-            raise ValueError(f"input on {x.device}, weights on {self.device}")
+                          words: Optional[Tuple[torch.Tensor, ...]] = None) -> torch.Tensor:
+        """fp16 ``x @ W.T`` through the packed transposed kernel, over the
+        matrix's packed tensors or those a forward saved.  The fp32 planes
+        are this call's own: one buffer for all calls would be shared by
+        streams, and growing it for a larger call would free what a captured
+        smaller one writes."""
+        qweight, qzeros, scales, perm = self._words() if words is None else words
+        device = qweight.device
+        if x.device != device:
+            raise ValueError(f"input on {x.device}, weights on {device}")
         if x.dtype != torch.float16:
             raise TypeError(f"the packed transposed kernel takes fp16, got {x.dtype}")
         outshape = x.shape[:-1] + (self.height,)
         g2 = _aligned_rows(x.reshape(-1, self.width))
         m = g2.shape[0]
-        out2 = torch.empty((m, self.height), dtype=torch.float16, device=self.device) \
+        out2 = torch.empty((m, self.height), dtype=torch.float16, device=device) \
             if output is None else _output_rows(output, m, self.height, torch.float16)
         nbytes = _lib.gemm_t_workspace_size(m, self.height, self.width, self.group_size)
-        ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=self.device) \
-            if own_workspace else self.cache.transpose_workspace(nbytes)
+        ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=device)
         _lib.call("dw4_gemm_t", m, self.height, self.width, self.group_size,
-                  g2.data_ptr(), g2.stride(0), self.qweight.data_ptr(), self.qzeros.data_ptr(),
-                  self.scales.data_ptr(), _ptr(self.perm) if self.use_act else None,
-                  out2.data_ptr(), out2.stride(0), ws.data_ptr(), ws.numel(), _stream(self.device))
+                  g2.data_ptr(), g2.stride(0), qweight.data_ptr(), qzeros.data_ptr(),
+                  scales.data_ptr(), _ptr(perm) if self.use_act else None,
+                  out2.data_ptr(), out2.stride(0), ws.data_ptr(), ws.numel(), _stream(device))
         return out2.view(outshape) if output is None else output
 
     def _dense_weight(self, temp_weight: Optional[torch.Tensor],
@@ -473,6 +471,15 @@ class Q4MatrixV2(object):
         if dtype == torch.bfloat16:
             return self.get_bfloat16_weights_matrix_v2(w)
         return self.get_float16_weights_matrix_v2(w)
+
+    def _dequantised(self, words: Tuple[torch.Tensor, ...]) -> torch.Tensor:
+        """The fp16 weight of packed tensors that a forward saved, in a buffer of its own."""
+        qweight, qzeros, scales, perm = words
+        w = torch.empty(self.height, self.width, dtype=torch.float16, device=qweight.device)
+        _lib.call("dw4_dequant", self.height, self.width, self.group_size, qweight.data_ptr(),
+                  qzeros.data_ptr(), scales.data_ptr(), _ptr(perm) if self.use_act else None,
+                  w.data_ptr(), w.stride(0), _stream(qweight.device))
+        return w
 
     def get_float16_weights_matrix_v2(self, out_matrix: Optional[torch.Tensor] = None) -> torch.Tensor:
         """Dequantised fp16 weight [K, N] in the checkpoint's row order."""
@@ -559,7 +566,7 @@ class Q4MatrixV2(object):
             return self._transpose_native(x, output)
         if w is None and not skip_reconstruct and temp_weight is None and output is None \
                 and x.device == self.device and _untracked(x) and self._packed_rows(m, dtype):
-            return self._transpose_native(x, None, own_workspace=True)
+            return self._transpose_native(x, None)
         if w is None:
             if skip_reconstruct:
                 if temp_weight is None:
@@ -581,12 +588,15 @@ class Q4LinearFunction(Function):
     """Frozen quantised weight; only the activation receives a gradient.
 
     As ``ExllamaQ4LinearFunction`` (``exllama.py:649-696``): with
-    ``cache_weight`` the dequantised weight of the input's dtype is kept for
-    the backward, unless the matrix already holds a reconstructed one or the
-    backward runs on the packed words (fp16 rows up to the library's rule,
+    ``cache_weight`` the dequantised weight of the input's dtype is saved for
+    the backward (unless the matrix already holds a reconstructed one).  Where
+    the backward runs on the packed words (fp16 rows up to the library's rule,
     where writing the dense weight costs more than it saves: 128 rows on
-    4096 x 11008 74 us to write and use, against 29 packed);
-    the forward of fp16 input still runs the W4A16 kernel, bf16 input the
+    4096 x 11008 74 us to write and use, against 29 packed), the packed
+    tensors are saved in its place, so the gradient is that of the forward's
+    weight whatever the matrix has been pointed at since, and autograd
+    refuses it if they were overwritten.
+    The forward of fp16 input still runs the W4A16 kernel, bf16 input the
     dense product over the kept weight.
     """
 
@@ -594,37 +604,42 @@ class Q4LinearFunction(Function):
     def forward(ctx: Any, input: torch.Tensor, weight_q4: Q4MatrixV2,  # type: ignore[override]
                 bias: Optional[torch.Tensor], cache_weight: bool) -> torch.Tensor:
         ctx.weight_q4 = weight_q4
+        ctx.kept = None
         cached = None
-        ctx.own_weight = cache_weight and weight_q4._reconstructed(input.dtype) is None
-        if ctx.own_weight and not weight_q4.packed_transpose(input):
-            cached = weight_q4._dense_weight(
-                torch.empty(weight_q4.height * weight_q4.width, dtype=input.dtype,
-                            device=weight_q4.device), input.dtype)
+        if cache_weight and weight_q4._reconstructed(input.dtype) is None:
+            if weight_q4.packed_transpose(input):
+                ctx.kept = "packed"
+                ctx.save_for_backward(*weight_q4._words())
+            else:
+                ctx.kept = "dense"
+                cached = weight_q4._dense_weight(
+                    torch.empty(weight_q4.height * weight_q4.width, dtype=input.dtype,
+                                device=weight_q4.device), input.dtype)
+                ctx.save_for_backward(cached)
         if cached is not None and input.dtype == torch.bfloat16:
-            output = weight_q4.matmul(input, temp_weight=cached, must_blas=True, bias=bias)
-        else:
-            output = weight_q4.matmul(input, bias=bias)
-        if cached is not None:
-            ctx.save_for_backward(cached)
-        ctx.has_cached = cached is not None
-        return output
+            return weight_q4.matmul(input, temp_weight=cached, must_blas=True, bias=bias)
+        return weight_q4.matmul(input, bias=bias)
 
     @staticmethod
     def backward(ctx: Any, grad_output: torch.Tensor):  # type: ignore[override]
         grad_input = None
         if ctx.needs_input_grad[0]:
-            if ctx.has_cached:
-                grad_input = ctx.weight_q4.transpose_matmul(
-                    grad_output, None, ctx.saved_tensors[0], skip_reconstruct=True)
-            elif ctx.own_weight and not _untracked(grad_output):
-                # recorded or transformed: the dense product over a weight of
-                # its own, which a later backward of this one may read
-                q4 = ctx.weight_q4
-                own = q4._dense_weight(torch.empty(q4.height * q4.width, dtype=grad_output.dtype,
-                                                   device=q4.device), grad_output.dtype)
-                grad_input = q4.transpose_matmul(grad_output, None, own, skip_reconstruct=True)
+            q4 = ctx.weight_q4
+            if ctx.kept == "packed":
+                q4._check_resident()
+                words = ctx.saved_tensors
+                if _untracked(grad_output):
+                    grad_input = q4._transpose_native(grad_output, None, words)
+                else:
+                    # recorded or transformed: the dense product over a weight of
+                    # its own, which a later backward of this one may read
+                    grad_input = q4.transpose_matmul(grad_output, None, q4._dequantised(words),
+                                                     skip_reconstruct=True)
+            elif ctx.kept == "dense":
+                grad_input = q4.transpose_matmul(grad_output, None, ctx.saved_tensors[0],
+                                                 skip_reconstruct=True)
             else:
-                grad_input = ctx.weight_q4.transpose_matmul(grad_output)
+                grad_input = q4.transpose_matmul(grad_output)
         return grad_input, None, None, None
 
 

@@ -218,3 +218,88 @@ def test_backward_with_kept_weight(hip_device, m):
     q4.cache.temp_weight.zero_()
     ddy, = torch.autograd.grad(dx2, tracked, x.detach())
     _check(ddy, x.detach().cpu(), w.T, "second order")
+
+
+def _trained(q4, m, seed):
+    x = make_x(m, q4.height, seed=seed).to(q4.device).requires_grad_(True)
+    dy = make_x(m, q4.width, seed=seed + 1).to(q4.device)
+    return x, dy
+
+
+def _step(q4, x, dy, kept=True):
+    y = Q4LinearFunction.apply(x, q4, None, kept)
+    return torch.autograd.grad(y, x, dy)[0]
+
+
+def test_captured_backward_owns_its_planes(hip_device):
+    """A forward and backward of 8 rows captured, then larger backwards through
+    the same cache, which once shared one buffer of planes, freed as it grew."""
+    lay, w = _layer(1152, 1056, 128, 8600, True)
+    q4 = _matrix(lay, hip_device)
+    q4.tuning_params = TuningParams(MAX_M=256)
+    assert _lib.gemm_t_workspace_size(8, 1152, 1056, 128) > 0  # planes there are
+    x, dy = _trained(q4, 8, 8601)
+    say("captured forward and backward of 8 rows, larger ones between the replays")
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        want = _step(q4, x, dy)
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = _step(q4, x, dy)
+    for i, m in enumerate((64, 100, 128)):
+        got.fill_(float("nan"))
+        graph.replay()
+        big, dbig = _trained(q4, m, 8610 + i)
+        dx = _step(q4, big, dbig)
+        fill = [torch.full((1 << 18,), float(i), device=hip_device) for _ in range(8)]
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
+        assert all(bool((f == i).all()) for f in fill)
+        _check(dx, dbig.cpu(), w, f"eager backward of {m} rows")
+
+
+def test_backwards_on_two_streams(hip_device):
+    lay, _ = _layer(1152, 1056, 128, 8600, True)
+    q4 = _matrix(lay, hip_device)
+    q4.tuning_params = TuningParams(MAX_M=256)
+    grads = [_trained(q4, m, 8620 + m)[1] for m in (8, 100)]
+    want = [q4.transpose_matmul(g) for g in grads]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in grads]
+    say("transposed products on two streams")
+    outs = [[], []]
+    for _ in range(20):
+        for i, st in enumerate(streams):
+            with torch.cuda.stream(st):
+                outs[i].append(q4.transpose_matmul(grads[i]))
+    torch.cuda.synchronize()
+    for i in range(2):
+        assert all(torch.equal(o, want[i]) for o in outs[i])
+
+
+def test_kept_backward_is_of_the_forwards_words(hip_device):
+    """The matrix pointed at other words, or its limit changed, between the
+    forward and the backward: the gradient stays that of the forward; words
+    overwritten in place are refused."""
+    lay, w = _layer(1152, 1056, 128, 8600, True)
+    q4 = _matrix(lay, hip_device)
+    q4.tuning_params = TuningParams(MAX_M=256)
+    x, dy = _trained(q4, 24, 8630)
+    say("backward after rebind, after a new limit, after an overwrite")
+    y = Q4LinearFunction.apply(x, q4, None, True)
+    words = [t.clone() for t in q4._words()]
+    q4.rebind(torch.zeros_like(words[0]), *words[1:])
+    _check(torch.autograd.grad(y, x, dy)[0], dy.cpu(), w, "rebound")
+    q4.rebind(*words)
+    y = Q4LinearFunction.apply(x, q4, None, True)
+    q4.set_tuning_params(TuningParams(MAX_M=256, TRANSPOSE_MAX_M=0))
+    _check(torch.autograd.grad(y, x, dy)[0], dy.cpu(), w, "new limit")
+    q4.set_tuning_params(TuningParams(MAX_M=256))
+    y = Q4LinearFunction.apply(x, q4, None, True)
+    q4.qweight.zero_()
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        torch.autograd.grad(y, x, dy)
