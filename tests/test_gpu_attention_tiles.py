@@ -117,3 +117,39 @@ def test_infinite_value_stays_infinite(hip_device):
     # fp32 sums of 128 products to 35: logits off by 2^-16 at most, outputs by twice that of max|v|
     err = np.abs(got[~inf] - ref[~inf])
     assert np.all(err <= 2.0 ** -11 * np.abs(ref[~inf]) + 2.0 ** -15 * 6), float(err.max())
+
+
+@pytest.mark.parametrize("heads,kvh,hs,bs", [(16, 2, 128, 16), (8, 2, 64, 32), (6, 2, 256, 16)])
+def test_probabilities_keep_their_bits(hip_device, heads, kvh, hs, bs):
+    """Two tokens, each with a one in a dim of its own: the partition's fp32
+    sums are then the two probabilities themselves, 1 and p, and its sum of
+    them is 1 + p rounded once, to the bit.  (Two fp16 parts of p, 21 bits
+    cut downwards, miss the sum in one case of five.)"""
+    say(f"probabilities heads={heads}/{kvh} hs={hs} bs={bs}")
+    n, ctx_max = 30, 600
+    rng = np.random.default_rng(hs)
+    kc = np.zeros((n, kvh, hs // 8, bs, 8), np.float16)
+    kc[:, :, :, 1, :] = rng.standard_normal((n, kvh, hs // 8, 8))
+    vc = np.zeros((n, kvh, hs, bs), np.float16)
+    vc[:, :, 0, 0] = vc[:, :, 1, 1] = 1
+    q = rng.standard_normal((n, heads, hs)).astype(np.float16)
+    tables = np.zeros((n, (ctx_max + bs - 1) // bs), np.int32)
+    tables[:, 0] = np.arange(n)
+    dev = lambda a: torch.from_numpy(a).to(hip_device)  # noqa: E731
+    kd, vd, qd, tab = dev(kc), dev(vc), dev(q), dev(tables)
+    ptrs = [torch.tensor([t[i].data_ptr() for i in range(n)], dtype=torch.int64, device=hip_device)
+            for t in (kd, vd)]
+    lens = torch.full((n,), 2, dtype=torch.int32, device=hip_device)
+    out = torch.empty(n, heads, hs, dtype=torch.float16, device=hip_device)
+    nbytes = _lib.paged_attention_workspace_size(n, heads, kvh, hs, bs, ctx_max)
+    parts = nbytes // (4 * n * heads * (2 + hs))
+    assert parts > 1  # partial results in the workspace: (max, sum), then the outputs
+    ws = torch.full((nbytes // 4,), float("nan"), device=hip_device)
+    _lib.call("dw4_paged_attention", n, heads, kvh, hs, bs, qd.data_ptr(), heads * hs, out.data_ptr(), heads * hs,
+              ptrs[0].data_ptr(), ptrs[1].data_ptr(), hs * bs, hs ** -0.5, tab.data_ptr(), tables.shape[1],
+              lens.data_ptr(), ctx_max, None, ws.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream)
+    rows = n * heads * parts
+    ml = ws[:2 * rows].view(n, heads, parts, 2)[:, :, 0].cpu().numpy()
+    o = ws[2 * rows:].view(n, heads, parts, hs)[:, :, 0, :2].cpu().numpy()
+    assert (o.max(axis=2) == 1).all() and (o.min(axis=2) > 0).all()
+    assert np.array_equal(o[..., 0] + o[..., 1], ml[..., 1])
