@@ -231,8 +231,9 @@ dw4::PrefillPlan plan_stream(int m, int k, int n, int count, int split_req, size
       const int cps = (kc + s - 1) / s;
       const int splits = (kc + cps - 1) / cps;
       if (split_req <= 0 && s > 1 && (cps < kStreamMinChunks || splits != s)) break;
-      // the caller's planes do not fit: that call runs unsplit
-      const bool fits = splits == 1 || stream_ws_bytes(splits, m32, n) <= ws_bytes;
+      // the caller's planes do not fit: that call runs unsplit.  They are
+      // the planes of the m rows, as sized (workspace_for) and as written.
+      const bool fits = splits == 1 || stream_ws_bytes(splits, m, n) <= ws_bytes;
       if (!fits && split_req <= 0) break;
       const int real = fits ? splits : 1;
       const int chunks = real == splits ? cps : kc;
@@ -268,6 +269,18 @@ constexpr int kStreamMinMAct = 65;
 
 bool use_stream(int m, int64_t ldx, bool act) {
   return m >= (act ? kStreamMinMAct : kStreamMinM) && dw4::prefill_x_fits(ldx);
+}
+
+// The plan of one streamed call in `room` bytes of workspace.  Act-order: the
+// gathered rows come first; a split only with what is left (in whole 256
+// bytes, as gather_offset aligns the rows after it).
+dw4::PrefillPlan plan_stream_in(int m, int k, int n, int split_req, bool act, size_t room,
+                                double* cost = nullptr) {
+  if (act) {
+    const size_t need = dw4::gather_bytes(m, k);
+    room = room > need ? (room - need) & ~(size_t)255 : 0;
+  }
+  return plan_stream(m, k, n, 1, split_req, room, cost);
 }
 
 hipError_t launch_stream(const dw4::GroupArgs& g, const dw4::PrefillPlan& plan, void* ws,
@@ -367,6 +380,27 @@ int dw4_workspace_size(int m, int k, int n, int group_size, int act_order, size_
   if (st != DW4_OK) return st;
   if (m < 0 || workspace_bytes == nullptr) return DW4_ERR_INVALID_ARG;
   *workspace_bytes = workspace_for(DW4_PATH_AUTO, m, k, n, group_size, act_order != 0);
+  return DW4_OK;
+}
+
+int dw4_prefill_plan(int m, int k, int n, int group_size, int act_order, size_t workspace_bytes,
+                     dw4_prefill_info* info) {
+  const int st = check_shape(k, n, group_size);
+  if (st != DW4_OK) return st;
+  if (m < 1 || info == nullptr) return DW4_ERR_INVALID_ARG;
+  const bool act = act_order != 0;
+  dw4::PrefillPlan p;
+  *info = dw4_prefill_info{};
+  if (use_stream(m, 0, act) && (!act || workspace_bytes >= dw4::gather_offset(0) + dw4::gather_bytes(m, k))) {
+    p = plan_stream_in(m, k, n, 0, act, workspace_bytes, &info->model_us);
+    info->kernel = p.kslice ? DW4_PREFILL_K_SLICED : DW4_PREFILL_LDS_STREAMED;
+  } else {
+    p = plan_prefill(m, k, n, 0, workspace_bytes, true);
+    info->kernel = DW4_PREFILL_REGISTER_FED;
+  }
+  info->tile_rows = p.bm;
+  info->tile_cols = p.bn;
+  info->splits = p.splits;
   return DW4_OK;
 }
 
@@ -500,11 +534,7 @@ int gemm_run(int path, int split_k, int m, int k, int n, int group_size, const u
   // order; otherwise the register-fed ones, which gather per workgroup.
   const size_t room = workspace && aligned16(workspace) ? workspace_bytes : 0;
   if (use_stream(m, ldx, perm != nullptr)) {
-    dw4::PrefillPlan plan;
-    // act-order: the gathered rows come first; a split only with what is
-    // left (whole 256 bytes, as gather_offset aligns the rows after it)
-    const size_t need = perm != nullptr ? dw4::gather_bytes(m, k) : 0;
-    plan = plan_stream(m, k, n, 1, split_k, room > need ? (room - need) & ~(size_t)255 : 0);
+    const dw4::PrefillPlan plan = plan_stream_in(m, k, n, split_k, perm != nullptr, room);
     const int e = gather_after(plan.splits > 1 ? stream_ws_bytes(plan.splits, m, n) : 0);
     if (e != DW4_OK) return e;
     if (a.perm == nullptr) {
@@ -612,9 +642,7 @@ int dw4_gemm_bf16_prefill(int m, int k, int n, int group_size, const uint16_t* x
   // bf16) after the planes; the kernels do not gather themselves
   const size_t gather = perm != nullptr ? dw4::gather_bytes(m, k) : 0;
   if (perm != nullptr && room < dw4::gather_offset(0) + gather) return DW4_ERR_WORKSPACE;
-  // (whole 256 bytes, as gather_offset aligns the rows after the planes)
-  dw4::PrefillPlan plan =
-      plan_stream(m, k, n, 1, 0, room > gather ? (room - gather) & ~(size_t)255 : 0);
+  dw4::PrefillPlan plan = plan_stream_in(m, k, n, 0, perm != nullptr, room);
   plan.bf16 = true;
   dw4::GroupArgs g{};
   g.count = 1;

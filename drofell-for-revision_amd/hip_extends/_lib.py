@@ -64,6 +64,13 @@ class ChainPlan(ctypes.Structure):
                 ("smem_bytes", _c.c_size_t)]
 
 
+class PrefillInfo(ctypes.Structure):
+    """``dw4_prefill_info``: the plan of one prefill call."""
+
+    _fields_ = [("kernel", _c.c_int), ("tile_rows", _c.c_int), ("tile_cols", _c.c_int),
+                ("splits", _c.c_int), ("model_us", _c.c_double)]
+
+
 _CLP = _c.POINTER(ChainLink)
 _CPP = _c.POINTER(ChainPlan)
 
@@ -94,6 +101,8 @@ SIGNATURES = {
     "dw4_stream_read": (_c.c_int, [_P, _c.c_size_t, _c.c_int, _c.c_int, _c.c_uint32, _P, _P]),
     "dw4_gemm_t": (_c.c_int, [_c.c_int, _c.c_int, _c.c_int, _c.c_int, _P, _c.c_int64, _P, _P, _P,
                               _P, _P, _c.c_int64, _P, _c.c_size_t, _P]),
+    "dw4_prefill_plan": (_c.c_int, [_c.c_int, _c.c_int, _c.c_int, _c.c_int, _c.c_int, _c.c_size_t,
+                                    _c.POINTER(PrefillInfo)]),
     "dw4_gemm_t_packed": (_c.c_int, [_c.c_int, _c.c_int, _c.c_int, _c.c_int,
                                      _c.POINTER(_c.c_int)]),
     "dw4_gemm_t_workspace_size": (_c.c_int, [_c.c_int, _c.c_int, _c.c_int, _c.c_int,
@@ -202,6 +211,14 @@ def workspace_size(m: int, k: int, n: int, group_size: int, act_order: bool) -> 
     check("dw4_workspace_size", lib.dw4_workspace_size(m, k, n, group_size, int(act_order),
                                                        ctypes.byref(out)))
     return out.value
+
+
+def prefill_plan(m: int, k: int, n: int, group_size: int, act_order: bool,
+                 workspace_bytes: int) -> PrefillInfo:
+    info = PrefillInfo()
+    check("dw4_prefill_plan", load().dw4_prefill_plan(m, k, n, group_size, int(act_order),
+                                                      workspace_bytes, ctypes.byref(info)))
+    return info
 
 
 def bf16_prefill_max_m(k: int, n: int, act_order: bool) -> int:

@@ -140,7 +140,8 @@ int dw4_query_sizes(int k, int n, int group_size, int act_order, int max_m,
  * it returns 0).  With act_order it includes M*K fp16 for x gathered into
  * the packed row order (placed after the split-K area and the arrival
  * counters); a call whose workspace lacks that room gathers inside every
- * workgroup instead: the same result bit for bit, slower.  (At M = 1 with
+ * workgroup instead, slower: up to 64 rows the same result bit for bit, above
+ * on another kernel, which sums in another order.  (At M = 1 with
  * K <= 16384 the decode kernel gathers from an LDS copy of x and uses none
  * of the act-order room.)  For 5 <= M <= 64
  * the decode kernel may split K over workgroups (fp32 planes in the
@@ -148,6 +149,26 @@ int dw4_query_sizes(int k, int n, int group_size, int act_order, int max_m,
  * result, summed in another order). */
 int dw4_workspace_size(int m, int k, int n, int group_size, int act_order,
                        size_t* workspace_bytes);
+
+/* The kernel, output tile and K split that a call on DW4_PATH_PREFILL takes at
+ * this M in a workspace of this size (x rows at most 2^22 elements apart, split
+ * left to the library), for tests and benchmarks.  The plan in
+ * dw4_workspace_size(m, ...) or dw4_query_sizes(max_m >= m) bytes is the plan
+ * with unlimited room.  model_us: the time the choice was made by, in
+ * microseconds (0 for the register-fed kernels, whose plan has no model). */
+enum {
+  DW4_PREFILL_REGISTER_FED = 0,
+  DW4_PREFILL_LDS_STREAMED = 1,
+  DW4_PREFILL_K_SLICED = 2
+};
+typedef struct {
+  int kernel;
+  int tile_rows, tile_cols;
+  int splits;
+  double model_us;
+} dw4_prefill_info;
+int dw4_prefill_plan(int m, int k, int n, int group_size, int act_order, size_t workspace_bytes,
+                     dw4_prefill_info* info);
 
 /* Host: stable counting sort of rows by group (perm[new] = old) and its
  * validation.  g_idx_host, perm_host: int32 [k] host arrays. */

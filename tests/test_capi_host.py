@@ -375,3 +375,33 @@ def test_chain_prepare_validates_before_touching_a_device():
     assert prepare([link(bufs[0], bufs[1], group_size=64)]) == _lib.DW4_ERR_UNSUPPORTED
     assert prepare([link(bufs[0], bufs[1], k=16512, ldx=16512)]) == _lib.DW4_ERR_UNSUPPORTED
     assert lib.dw4_gemm_chain(None, None, None) == _lib.DW4_ERR_INVALID_ARG
+
+
+@pytest.mark.parametrize("act", [False, True], ids=["plain", "act"])
+def test_sized_workspace_holds_the_planned_split(act):
+    """The prefill plan in the bytes that were asked for (for this M, or for
+    any M up to a maximum) is the plan with unlimited room: sized, checked
+    and written for the same rows, whatever M and N are."""
+    free = (1 << 64) - 1
+
+    def key(m, k, n, room):
+        p = _lib.prefill_plan(m, k, n, 128, act, room)
+        return p.kernel, p.tile_rows, p.tile_cols, p.splits, p.model_us
+
+    split = 0
+    for k, n, step in ((11008, 4096, 1), (13824, 5120, 1), (5120, 5120, 1), (4096, 4096, 3),
+                       (4096, 11008, 3), (5120, 13824, 3), (4096, 8208, 1), (5120, 1040, 1)):
+        most = _lib.query_sizes(k, n, 128, act, 1000)["workspace"]
+        for m in range(33, 1001, step):
+            want = key(m, k, n, free)
+            split += want[3] > 1
+            assert key(m, k, n, most) == want, (m, k, n)
+            # DW4_PATH_AUTO may size a decode call instead
+            if _lib.workspace_size(m, k, n, 128, act) > 0 and m > 64:
+                assert key(m, k, n, _lib.workspace_size(m, k, n, 128, act)) == want, (m, k, n)
+        for m in (65, 100, 130, 449, 513, 641, 1000):
+            own = _lib.query_sizes(k, n, 128, act, m)["workspace"]
+            assert key(m, k, n, own) == key(m, k, n, free), (m, k, n)
+    assert split > 100
+    with pytest.raises(_lib.W4A16Error):
+        _lib.prefill_plan(0, 4096, 4096, 128, act, 0)

@@ -1,7 +1,7 @@
 """GPU parity of the prefill kernels' tiles at their edges: every tile of the
-K-sliced and the LDS-streamed kernel (a comment names the one a case's plan
-takes on 256 CUs) with partial row and column tiles, fewer chunks than waves,
-K splits, every group size form, act-order with and without room for the
+K-sliced and the LDS-streamed kernel (a case names its plan on 256 CUs, and
+the test asserts it) with partial row and column tiles, fewer chunks than
+waves, K splits, every group size form, act-order with and without room for the
 gathered rows, fp16 and bf16 activations, strided and unaligned rows, and the
 grouped launch.
 
@@ -63,30 +63,31 @@ def _check(y, x, w, bias, what):
         f"{what}: worst error / bound {np.nanmax(err / bound):.3f}"
 
 
+# the plan on 256 CUs: K-sliced or LDS-streamed, tile, K splits
 CASES = [
-    # m, k, n, group, act
-    (33, 256, 80, 128, False),      # K-sliced 64 x 32, two chunks for eight waves
-    (64, 640, 400, 32, False),      # the same, 25 strips (the last column tile half full)
-    (97, 5120, 1040, 128, False),   # the same, three K splits
-    (65, 640, 4112, 64, False),     # K-sliced 32 x 64, five chunks
-    (65, 4096, 1040, 4096, False),  # K-sliced 64 x 32, two splits, one group
-    (33, 1024, 8208, 32, False),    # K-sliced 64 x 64
-    (97, 1024, 4112, 256, True),    # the same, act-order
-    (130, 5120, 1040, 256, True),   # K-sliced 64 x 32, two splits, act-order
-    (97, 256, 4112, 128, False),    # LDS-streamed 32 x 128
-    (130, 384, 8208, 64, False),    # 64 x 128
-    (97, 4096, 8208, 128, False),   # 64 x 256, three splits
-    (300, 256, 8208, 32, True),     # 32 x 128, act-order
-    (700, 1024, 8208, 128, False),  # 128 x 256
-    (600, 256, 8208, 128, False),   # 96 x 256
-    (385, 512, 8208, 64, False),    # 64 x 256, one row in the last tile
-    (1300, 384, 4112, 32, False),   # 96 x 256
+    # m, k, n, group, act, plan
+    (33, 256, 80, 128, False, "K 64x32/1"),      # two chunks for eight waves
+    (64, 640, 400, 32, False, "K 64x32/1"),      # 25 strips (the last column tile half full)
+    (97, 5120, 1040, 128, False, "K 64x32/3"),
+    (65, 640, 4112, 64, False, "K 32x64/1"),     # five chunks
+    (65, 4096, 1040, 4096, False, "K 64x32/2"),  # one group
+    (33, 1024, 8208, 32, False, "K 64x64/1"),
+    (97, 1024, 4112, 256, True, "K 64x64/1"),
+    (130, 5120, 1040, 256, True, "K 64x32/2"),
+    (97, 256, 4112, 128, False, "L 32x128/1"),
+    (130, 384, 8208, 64, False, "L 64x128/1"),
+    (97, 4096, 8208, 128, False, "L 64x256/3"),
+    (300, 256, 8208, 32, True, "L 32x128/1"),
+    (700, 1024, 8208, 128, False, "L 128x256/1"),
+    (600, 256, 8208, 128, False, "L 96x256/1"),
+    (385, 512, 8208, 64, False, "L 64x256/1"),   # one row in the last tile
+    (1300, 384, 4112, 32, False, "L 96x256/1"),
 ]
 
 
-@pytest.mark.parametrize("m,k,n,g,act", CASES)
+@pytest.mark.parametrize("m,k,n,g,act,plan", CASES)
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["fp16", "bf16"])
-def test_prefill_tiles(hip_device, m, k, n, g, act, dtype):
+def test_prefill_tiles(hip_device, m, k, n, g, act, plan, dtype):
     q4, w = _build(k, n, g, act, hip_device, m)
     x = _x(m, k, dtype, m)
     xd = x.to(hip_device)
@@ -104,6 +105,9 @@ def test_prefill_tiles(hip_device, m, k, n, g, act, dtype):
         y = torch.full((m, n + pad_y), float("nan"), dtype=dtype, device=hip_device)
         planes = 16384 + 4 * m * n * 4 + 512 + 2 * m * k
         ws = torch.zeros(max(16, room, planes if split else 0), dtype=torch.uint8, device=hip_device)
+        if split == 0:
+            p = _lib.prefill_plan(m, k, n, g, act, ws.numel())
+            assert f"{'RLK'[p.kernel]} {p.tile_rows}x{p.tile_cols}/{p.splits}" == plan
         args = (m, k, n, g, xs.data_ptr(), xs.stride(0), q4.qweight.data_ptr(), q4.qzeros.data_ptr(),
                 q4.scales.data_ptr(), perm, bias.to(hip_device).data_ptr(), y.data_ptr(), y.stride(0),
                 ws.data_ptr(), ws.numel(), stream)
