@@ -33,6 +33,8 @@ struct PagedAttnPlan {
   int waves = 4;  // per workgroup: 4, or 8 (one head per kv head: 16) for one workgroup per
                   // (sequence, kv head)
 };
+// The least tokens of a partition with grouped heads, twice that above so long a context.
+constexpr int kAttnLeastPart = 128, kAttnShortContext = 2048;
 // The 8-wave form: contexts up to this many tokens in one partition.
 constexpr int kAttnWideMaxTokens = 4096;
 // Dynamic LDS of a paged-attention workgroup: the waves' outputs
@@ -49,6 +51,10 @@ inline size_t attn_row_smem_bytes(int hs, int part_tokens, int waves) {
 }
 PagedAttnPlan plan_paged_attention(int num_seqs, int num_heads, int num_kv_heads, int head_size,
                                    int block_size, int max_context_len, int cus);
+// Bytes that serve every call of at most so many sequences and so long a context (one query head
+// per kv head: this call).
+size_t paged_attention_ws_upto(int num_seqs, int num_heads, int num_kv_heads, int head_size,
+                               int block_size, int max_context_len, int cus);
 size_t paged_attention_ws_bytes(const PagedAttnPlan& p, int num_seqs, int num_heads,
                                 int head_size);
 hipError_t launch_paged_attention(const PagedAttnArgs& a, const PagedAttnPlan& p, float* ws,

@@ -940,7 +940,7 @@ PagedAttnPlan plan_paged_attention(int num_seqs, int num_heads, int num_kv_heads
   // at most 4096.  Measured (us, at least 16 tokens and four workgroups per CU
   // -> this): 1 x 4000 tokens, 8 kv heads 31.3 -> 12.1; 32 x 1000 28.2 -> 22.8;
   // 8 x 3000, 16 heads of 256 61.0 -> 54.4.
-  const int least = max_context_len > 2048 ? 256 : 128;
+  const int least = max_context_len > kAttnShortContext ? 2 * kAttnLeastPart : kAttnLeastPart;
   int parts = (cus + pairs - 1) / pairs;
   parts = std::max(1, std::min(parts, (max_context_len + least - 1) / least));
   int bpp = (blocks + parts - 1) / parts;
@@ -954,6 +954,29 @@ size_t paged_attention_ws_bytes(const PagedAttnPlan& p, int num_seqs, int num_he
                                 int head_size) {
   if (p.num_parts <= 1) return 0;
   return sizeof(float) * (size_t)num_seqs * num_heads * p.num_parts * (2 + (size_t)head_size);
+}
+
+// Fewer sequences or a shorter context can take more partitions than the
+// largest call does (which may be one workgroup per pair, with none), so with
+// grouped heads the size is a bound over all of them: seqs * parts is at most
+// cus / kv_heads + seqs by the workgroups wanted, seqs times the most
+// partitions of any context up to this one by their least size, and seqs times
+// the partitions of 4096 tokens.
+size_t paged_attention_ws_upto(int num_seqs, int num_heads, int num_kv_heads, int head_size,
+                               int block_size, int max_context_len, int cus) {
+  if (num_seqs == 0) return 0;
+  if (num_heads == num_kv_heads)
+    return paged_attention_ws_bytes(plan_paged_attention(num_seqs, num_heads, num_kv_heads, head_size,
+                                                         block_size, max_context_len, cus),
+                                    num_seqs, num_heads, head_size);
+  auto ceil_of = [](int a, int b) { return a / b + (a % b != 0); };
+  int most = ceil_of(std::min(max_context_len, kAttnShortContext), kAttnLeastPart);
+  if (max_context_len > kAttnShortContext)
+    most = std::max(most, ceil_of(max_context_len, 2 * kAttnLeastPart));
+  const int64_t wanted = std::min((int64_t)num_seqs * most, (int64_t)ceil_of(cus, num_kv_heads) + num_seqs);
+  const int64_t full = (int64_t)num_seqs * ceil_of(max_context_len, kAttnMaxPartTokens);
+  const int64_t rows = std::max(wanted, full);
+  return most <= 1 ? 0 : sizeof(float) * (size_t)rows * num_heads * (2 + (size_t)head_size);
 }
 
 hipError_t launch_paged_attention(const PagedAttnArgs& a, const PagedAttnPlan& p, float* ws,

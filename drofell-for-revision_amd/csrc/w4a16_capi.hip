@@ -780,9 +780,8 @@ int dw4_paged_attention_workspace_size(int num_seqs, int num_heads, int num_kv_h
                                   max_context_len);
   if (st != DW4_OK) return st;
   if (workspace_bytes == nullptr) return DW4_ERR_INVALID_ARG;
-  const dw4::PagedAttnPlan p = dw4::plan_paged_attention(num_seqs, num_heads, num_kv_heads, head_size, block_size,
-                                                         max_context_len, cu_count());
-  *workspace_bytes = num_seqs == 0 ? 0 : dw4::paged_attention_ws_bytes(p, num_seqs, num_heads, head_size);
+  *workspace_bytes = dw4::paged_attention_ws_upto(num_seqs, num_heads, num_kv_heads, head_size, block_size,
+                                                  max_context_len, cu_count());
   return DW4_OK;
 }
 

@@ -430,7 +430,9 @@ int dw4_restore_from_cache(int num_tokens, int num_kv_heads, int head_size, int 
  * multiple of num_kv_heads with at most 8 query heads per kv head.
  * Softmax and both products in fp32; long contexts are split into
  * partitions combined in a fixed order (deterministic).  workspace: at
- * least dw4_paged_attention_workspace_size bytes (0 for short contexts).
+ * least dw4_paged_attention_workspace_size bytes (0 for short contexts); with
+ * several query heads per kv head these serve fewer sequences and shorter
+ * contexts too.
  * Never synchronises or allocates.  Replaces paged_attention_v1 / v2
  * (cuda_extends/vllm/attention/attention_kernels.cu:1602-1632, 1786-1843)
  * as operators/core/attention/real_page.py:23-189 calls them. */

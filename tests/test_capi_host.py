@@ -405,3 +405,16 @@ def test_sized_workspace_holds_the_planned_split(act):
     assert split > 100
     with pytest.raises(_lib.W4A16Error):
         _lib.prefill_plan(0, 4096, 4096, 128, act, 0)
+
+
+@pytest.mark.parametrize("heads,kvh,hs,bs", [(32, 8, 128, 32), (32, 8, 128, 16), (8, 2, 64, 16),
+                                             (16, 4, 256, 16), (64, 8, 80, 32)])
+def test_grouped_attention_workspace_grows_with_the_call(heads, kvh, hs, bs):
+    """More sequences or a longer context never ask for less, so the bytes of
+    the largest call serve the others."""
+    ctxs = (1, 16, 128, 129, 600, 1024, 1025, 2048, 2049, 2100, 3072, 4096, 4097, 9000, 40000)
+    size = [[_lib.paged_attention_workspace_size(s, heads, kvh, hs, bs, c) for c in ctxs]
+            for s in range(1, 200)]
+    assert all(a <= b for row in size for a, b in zip(row, row[1:]))
+    assert all(a <= b for lo, hi in zip(size, size[1:]) for a, b in zip(lo, hi))
+    assert size[0][0] == 0 and max(map(max, size)) < 64 << 20

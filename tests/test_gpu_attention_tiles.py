@@ -142,14 +142,49 @@ def test_probabilities_keep_their_bits(hip_device, heads, kvh, hs, bs):
     lens = torch.full((n,), 2, dtype=torch.int32, device=hip_device)
     out = torch.empty(n, heads, hs, dtype=torch.float16, device=hip_device)
     nbytes = _lib.paged_attention_workspace_size(n, heads, kvh, hs, bs, ctx_max)
-    parts = nbytes // (4 * n * heads * (2 + hs))
-    assert parts > 1  # partial results in the workspace: (max, sum), then the outputs
     ws = torch.full((nbytes // 4,), float("nan"), device=hip_device)
     _lib.call("dw4_paged_attention", n, heads, kvh, hs, bs, qd.data_ptr(), heads * hs, out.data_ptr(), heads * hs,
               ptrs[0].data_ptr(), ptrs[1].data_ptr(), hs * bs, hs ** -0.5, tab.data_ptr(), tables.shape[1],
               lens.data_ptr(), ctx_max, None, ws.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream)
+    # partial results: (max, sum) of every partition, then the outputs, of which
+    # only the first partition (the others hold no token) writes any
+    parts = (int((~torch.isnan(ws)).sum()) // (n * heads) - hs) // 2
+    assert parts > 1
     rows = n * heads * parts
     ml = ws[:2 * rows].view(n, heads, parts, 2)[:, :, 0].cpu().numpy()
-    o = ws[2 * rows:].view(n, heads, parts, hs)[:, :, 0, :2].cpu().numpy()
+    o = ws[2 * rows:rows * (2 + hs)].view(n, heads, parts, hs)[:, :, 0, :2].cpu().numpy()
     assert (o.max(axis=2) == 1).all() and (o.min(axis=2) > 0).all()
     assert np.array_equal(o[..., 0] + o[..., 1], ml[..., 1])
+
+
+@pytest.mark.parametrize("heads,kvh,hs,bs,most,calls", [
+    (32, 8, 128, 32, (32, 3072), [(1, 2048), (9, 1025), (32, 128)]),
+    (16, 4, 64, 16, (24, 4000), [(3, 600), (1, 2049), (1, 2048)]),
+    (8, 2, 256, 16, (5, 9000), [(4, 9000), (5, 2048), (1, 4097)])])
+def test_one_workspace_serves_smaller_calls(hip_device, heads, kvh, hs, bs, most, calls):
+    """A workspace of the size for the most sequences and the longest context
+    (which run as one workgroup per pair, without one) takes every call of
+    fewer or shorter ones."""
+    ws = torch.empty(max(16, _lib.paged_attention_workspace_size(most[0], heads, kvh, hs, bs, most[1])),
+                     dtype=torch.uint8, device=hip_device)
+    rng = np.random.default_rng(hs)
+    for n, ctx in calls:
+        say(f"attention {n} x {ctx} in the workspace of {most}")
+        per = (ctx + bs - 1) // bs
+        tables = rng.permutation(n * per).astype(np.int32).reshape(n, per)
+        kc = rng.standard_normal((n * per, kvh, hs // 8, bs, 8)).astype(np.float16)
+        vc = rng.standard_normal((n * per, kvh, hs, bs)).astype(np.float16)
+        q = rng.standard_normal((n, heads, hs)).astype(np.float16)
+        ctxs = rng.integers(1, ctx + 1, n)
+        ctxs[0] = ctx
+        ref = A.paged_attention(q, kc, vc, tables, ctxs, hs ** -0.5, None)
+        kd, vd, qd, tab = (torch.from_numpy(a).to(hip_device) for a in (kc, vc, q, tables))
+        ptrs = [torch.tensor([t[i].data_ptr() for i in range(n * per)], dtype=torch.int64, device=hip_device)
+                for t in (kd, vd)]
+        lens = torch.from_numpy(ctxs.astype(np.int32)).to(hip_device)
+        out = torch.empty(n, heads, hs, dtype=torch.float16, device=hip_device)
+        _lib.call("dw4_paged_attention", n, heads, kvh, hs, bs, qd.data_ptr(), heads * hs, out.data_ptr(),
+                  heads * hs, ptrs[0].data_ptr(), ptrs[1].data_ptr(), hs * bs, hs ** -0.5, tab.data_ptr(), per,
+                  lens.data_ptr(), ctx, None, ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream)
+        err = np.abs(out.cpu().numpy().astype(np.float64) - ref)
+        assert np.all(err <= 2.0 ** -11 * np.abs(ref) + 2.0 ** -17 * 6), float(err.max())
