@@ -14,7 +14,10 @@
 //     chunk of 64 k) and turned into MFMA operand order through the wave's own
 //     LDS region: 16-byte unit u of row r sits at u ^ (r & 7), so the stores
 //     and the operand reads are conflict-free, and a wave reads only what it
-//     wrote (LDS operations of one wave complete in order);
+//     wrote.  LDS operations of one wave complete in order, so no wait is
+//     needed, but lanes read what other lanes stored: wavefront fences keep
+//     the compiler from moving the reads over the stores or the next stores
+//     over the reads (they emit no instruction);
 //   * B operands as in the LDS-streamed kernel: two strips' packed words
 //     rearranged by permlane swaps, the exact fp16 weight fp16(s (q - z)), and
 //     v_mfma_f32_32x32x16_f16;
@@ -44,6 +47,13 @@ namespace dw4 {
 namespace {
 
 constexpr int kKsWaves = 8;
+
+// Orders the wave's LDS accesses before and after it (for the compiler: the
+// hardware keeps one wave's in order).
+__device__ __forceinline__ void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
 
 }  // namespace
 
@@ -196,9 +206,11 @@ kslice_kernel(const _Float16* __restrict__ x, int64_t ldx, int M, const P2Items 
       for (int h = 0; h < 2; ++h) {
         // (the compiler would sink the loads towards their uses)
         stage_a(h);
+        wave_fence();
         load_a(h, nx);
         __builtin_amdgcn_sched_barrier(0);
         compute(h);
+        wave_fence();
         __builtin_amdgcn_sched_barrier(0);
         load_b(h, nx);
         __builtin_amdgcn_sched_barrier(0);
