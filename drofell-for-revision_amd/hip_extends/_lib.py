@@ -171,13 +171,19 @@ def load(path: str = LIB_PATH) -> ctypes.CDLL:
         # streams from torch would belong to the other runtime).
         import torch  # noqa: F401
         lib = ctypes.CDLL(path)
+        # a library built from older sources: another ABI version, or entry
+        # points added since under the same one
+        version = lib.dw4_abi_version()
+        if version != ABI_VERSION:
+            raise RuntimeError(f"{LIB_NAME} ABI version {version}, expected {ABI_VERSION}")
+        missing = [name for name in SIGNATURES if not hasattr(lib, name)]
+        if missing:
+            raise RuntimeError(f"{LIB_NAME} at {path} is older than this package (ABI version "
+                               f"{version} without {', '.join(missing)}): build it again")
         for name, (res, args) in SIGNATURES.items():
             fn = getattr(lib, name)
             fn.restype = res
             fn.argtypes = args
-        version = lib.dw4_abi_version()
-        if version != ABI_VERSION:
-            raise RuntimeError(f"{LIB_NAME} ABI version {version}, expected {ABI_VERSION}")
         _lib = lib
         return lib
 

@@ -7,6 +7,7 @@ from __future__ import annotations
 import ctypes
 import os
 import re
+import subprocess
 
 import numpy as np
 import pytest
@@ -418,3 +419,16 @@ def test_grouped_attention_workspace_grows_with_the_call(heads, kvh, hs, bs):
     assert all(a <= b for row in size for a, b in zip(row, row[1:]))
     assert all(a <= b for lo, hi in zip(size, size[1:]) for a, b in zip(lo, hi))
     assert size[0][0] == 0 and max(map(max, size)) < 64 << 20
+
+
+@pytest.mark.parametrize("version,match", [(10, "ABI version 10, expected"), (11, "older than this package")])
+def test_stale_library_is_named(tmp_path, monkeypatch, version, match):
+    """A library of older sources is refused by what it is: by its ABI version,
+    or by the entry points it lacks, never by a failing symbol lookup."""
+    src = tmp_path / "stale.c"
+    src.write_text(f"int dw4_abi_version(void) {{ return {version}; }}\n")
+    so = tmp_path / "libstale.so"
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(so), str(src)], check=True)
+    monkeypatch.setattr(_lib, "_lib", None)
+    with pytest.raises(RuntimeError, match=match):
+        _lib.load(str(so))
