@@ -69,9 +69,10 @@ int status_of(hipError_t e) { return e == hipSuccess ? DW4_OK : DW4_ERR_LAUNCH; 
 size_t prefill_ws_bytes(const dw4::PrefillPlan& p, int m, int n);
 
 // Tiling and split-K factor of the register-fed prefill kernels
-// (launch_prefill): act-order calls whose workspace cannot hold the gathered
-// rows, x rows too far apart for 32-bit offsets, and M <= 32.  `ws_bytes`
-// caps the split count: with too little workspace the call runs unsplit.
+// (launch_prefill): M up to 32, act-order calls up to 64 rows or whose
+// workspace cannot hold the gathered rows, and x rows too far apart for 32-bit
+// offsets.  `ws_bytes` caps the split count: with too little workspace the
+// call runs unsplit.
 dw4::PrefillPlan plan_prefill(int m, int k, int n, int split_req, size_t ws_bytes, bool cap_by_ws) {
   dw4::PrefillPlan p;
   // Row tile: 16 or 32 rows just covering small M, then 64 (above 128 rows
@@ -99,15 +100,17 @@ dw4::PrefillPlan plan_prefill(int m, int k, int n, int split_req, size_t ws_byte
     p.bn = 128;
     if (p.bm == 64 && m <= 64 && filled(32, 128) > filled(64, 128)) p.bm = 32;
   }
-  // Above 128 rows, the LDS-streamed kernel, on the tile shape that needs
-  // the fewest rounds of workgroups (one workgroup per CU at a time), ties
-  // going to the first of: 64 x 256 (up to 512 rows: twice the tiles of
-  // 128-row ones, so fewer split-K partial planes), 128 x 128, 128 x 256
-  // (each dequantised weight fragment feeds four MFMAs in the 128-row
-  // tiles).  Measured (us): 4096^2 M=512 30.8 with 64 x 256 against 35.1
-  // with 128 x 128; 4096x11008 M=512 74.4 with two rounds of 64 x 256
-  // against 61.3 with one of 128 x 256; 4096^2 M=1024 42.0 with 128 x 128
-  // against 52.9 with 64 x 256.
+  // Above 128 rows the tile of the fewest rounds of workgroups (one per CU),
+  // ties going to the first of 64 x 256 (up to 512 rows), 128 x 128, 128 x
+  // 256; with K up to 4096, 64 x 128 up to 512 rows where it needs fewer K
+  // splits, and 32 x 128 up to 256 where two per CU hold all of them.  The
+  // K <= 4096 choices need the least workspace (dw4_workspace_size counts
+  // these planes); they are not the fastest tiles for the calls that come here.  Of
+  // these, act-order calls without room for the gathered rows gather in every
+  // workgroup, so that wide tiles are best (us, one workgroup's gathers per
+  // column tile): 4096 x 11008, 160 rows, 32 x 128 176, 64 x 256 125; 384 rows,
+  // 128 x 256 239, 64 x 256 277, 128 x 128 441; with room the same calls take 38
+  // and 55 on the streamed kernels.
   if (m > 128) {
     const int cand[3][2] = {{64, 256}, {128, 128}, {128, 256}};
     int best_rounds = 1 << 30;
@@ -120,11 +123,6 @@ dw4::PrefillPlan plan_prefill(int m, int k, int n, int split_req, size_t ws_byte
         p.bn = cand[c][1];
       }
     }
-    // 4-wave 64 x 128 workgroups (two per CU) where they need fewer K splits
-    // in as few rounds, for K up to 4096 (longer K keeps the 8-wave tiles,
-    // whose chunks run ~10 % faster).  Measured (us): 4096^2 M=256 24.4 ->
-    // 23.5 (2 splits instead of 4), M=384 28.3 -> 26.5, M=512 31.9 -> 28.2
-    // (unsplit); 11008x4096 M=384 57.4 against 61.5 with the 4-wave tiles.
     if (m <= 512 && kc <= 32) {
       const int t8 = ((m + p.bm - 1) / p.bm) * ((n + p.bn - 1) / p.bn);
       const int t4 = ((m + 63) / 64) * ((n + 127) / 128);
@@ -132,30 +130,18 @@ dw4::PrefillPlan plan_prefill(int m, int k, int n, int split_req, size_t ws_byte
       if ((t4 * s4 + 2 * cus_now - 1) / (2 * cus_now) <= best_rounds && s4 < s8) {
         p.bm = 64;
         p.bn = 128;
-        p.waves = 4;
       }
     }
-    // Up to 256 rows with K up to 4096: 4-wave 32 x 128 workgroups where
-    // they fit two per CU.  A 32-row chunk costs ~0.52 us against ~0.72 us
-    // for 64 x 128, so with K this short the extra dequantisation per row
-    // costs less than the split planes and reduce launch the taller tiles
-    // need.  Measured (us): 4096^2 M=160 22.4 -> 21.0, M=256 23.6 -> 21.4;
-    // 4096x11008 M=160 39.8 -> 34.2.
-    if (m <= 256 && kc <= 32) {
-      const int t32 = ((m + 31) / 32) * ((n + 127) / 128);
-      if (t32 <= 2 * cus_now) {
-        p.bm = 32;
-        p.bn = 128;
-        p.waves = 4;
-      }
+    if (m <= 256 && kc <= 32 && ((m + 31) / 32) * ((n + 127) / 128) <= 2 * cus_now) {
+      p.bm = 32;
+      p.bn = 128;
     }
   }
   const int tiles = ((m + p.bm - 1) / p.bm) * ((n + p.bn - 1) / p.bn);
   // Automatic splits: enough to give every CU a workgroup (one per CU at a
   // time), with at least 8 chunks per split and at most 8 splits: every
-  // split adds a partial plane to write and sum (the LDS-streamed kernel) or
-  // lengthens the last-arriving split's sum (the kernel below 129 rows)
-  // faster than it adds parallelism (measured on 7B shapes).
+  // split lengthens the last-arriving split's sum faster than it adds
+  // parallelism (measured on 7B shapes).
   int splits = split_req > 0 ? split_req : auto_splits(tiles);
   splits = std::max(1, std::min(splits, kc));
   // the launcher rounds to whole chunks per split

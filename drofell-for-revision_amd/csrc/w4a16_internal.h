@@ -81,8 +81,8 @@ struct Items {
   int count;
 };
 
-// Prefill launch: row tile bm (16: 16x16x32 MFMA kernel; 32, 64, 128:
-// 32x32x16 MFMA kernel), column tile bn (128 or 256), split-K factor.
+// Prefill launch: output tile bm x bn and split-K factor.  Register-fed
+// kernels: bm 16 (16x16x32 MFMA), 32, 64 or 128 (32x32x16), bn 128 or 256.
 struct PrefillPlan {
   int bm, bn, splits;
   int waves = 8;  // LDS-streamed kernel: 8 (one workgroup per CU) or 4 (two)
