@@ -20,6 +20,7 @@ import pytest
 import torch
 
 from gptq_synth import GPTQLayer, make_layer, make_x
+from hip_extends import _lib
 from hip_extends.w4a16 import (CacheV2, Q4MatrixV2, TuningParams,
                                decoder_after_stage_v2_py)
 from oracle import gptq, stage
@@ -46,14 +47,14 @@ def layer_w(k, n, g, seed, act, gidx_from=None):
     return lay, gptq.dequantize(a["qweight"], a["qzeros"], a["scales"], a["g_idx"])
 
 
-def build(layers, dev):
+def build(layers, dev, max_m=64):
     cache = CacheV2(dev)
     q4s = []
     for lay in layers:
         d = lay.to(dev)
         q4s.append(Q4MatrixV2(d.qweight, d.qzeros, d.scales, d.in_features, d.out_features,
                               d.g_idx if d.act_order else None, d.act_order,
-                              TuningParams(MAX_M=64), cache))
+                              TuningParams(MAX_M=max_m), cache))
     cache.init_cache()
     return q4s, cache
 
@@ -110,14 +111,18 @@ def _check_after(b, m, attn, res, ws, wn, what):
 def test_after_stage(hip_device, shape, act):
     hidden, inter = shape
     lws = _layers(hidden, inter, act, 1000 + hidden)
-    q4s, cache = build([lw[0] for lw in lws], hip_device)
+    q4s, cache = build([lw[0] for lw in lws], hip_device, 64 if act else 1024)
     if act:
         assert q4s[1].perm.data_ptr() == q4s[2].perm.data_ptr()  # gate/up share: chained
     ws = [lw[1] for lw in lws]
     wn = norm_weight(hidden, 7)
-    # 7B up to M=256: the LDS-streamed prefill tiles' residual epilogues
-    # (32 x 128 for o_proj, 64 x 256 with K splits and the reduce for down)
-    ms = (1, 2, 3, 4, 8) if act else (1, 2, 3, 4, 8, 16, 33, 64, 100, 200, 256)
+    # 7B up to M=256: the K-sliced tiles' residual epilogue; at 1024 rows the
+    # LDS-streamed one (64 x 256, o_proj) and the reduce's (down, two K splits)
+    ms = (1, 2, 3, 4, 8) if act else (1, 2, 3, 4, 8, 16, 33, 64, 100, 200, 256, 1024)
+    if not act:
+        room = cache.workspace.numel()
+        o, d = (_lib.prefill_plan(1024, q.height, q.width, 128, False, room) for q in (q4s[0], q4s[3]))
+        assert (o.kernel, o.splits, d.kernel, d.splits) == (1, 1, 1, 2)
     b = _Bufs(max(ms), hidden, inter, hip_device)
     for m in ms:
         say(f"after_stage {hidden}x{inter} act={act} M={m}")

@@ -267,10 +267,10 @@ def test_act_order_gather_first_matches_in_kernel_gather(hip_device):
     Where that is the same kernel (decode; prefill tiles below 256 columns)
     they feed the same values to the same sums and the outputs are
     bit-identical.
-    At M=300 the gathered rows go to the LDS-streamed 64 x 256 tile kernel,
-    whose two waves per column quarter sum alternate k halves and add them at
-    the end; the per-workgroup gather stays on the sequential-k kernel, so
-    there both are held to the oracle's tolerance instead."""
+    At M=300 the gathered rows go to the K-sliced 64 x 64 tile kernel, whose
+    waves each sum every eighth chunk and add up at the end; the per-workgroup
+    gather stays on the sequential-k kernel, so there both are held to the
+    oracle's tolerance instead."""
     k, n = 5120, 2048
     lay, w = oracle_w(k, n, 128, 4242, False, True)
     q4 = build(lay, hip_device)
@@ -358,7 +358,8 @@ def test_prefill_large_m_and_split_k(hip_device):
 @pytest.mark.parametrize("kn", SHAPES_7B, ids=lambda kn: f"{kn[0]}x{kn[1]}")
 def test_prefill_7b_large_m(hip_device, kn):
     """Config 3 at M = 1024 and 2048 on every 7B shape through the automatic
-    path (128 x 128 or 128 x 256 tiles of the LDS-streamed kernel)."""
+    path (64, 96 and 128 x 256 tiles of the LDS-streamed kernel, 11008 x 4096
+    at M = 1024 split in two)."""
     k, n = kn
     lay, w = oracle_w(k, n, 128, 1000 + SHAPES_7B.index(kn), False, False)
     q4 = build(lay, hip_device)
@@ -384,14 +385,14 @@ def test_prefill_7b_large_m(hip_device, kn):
                               "4096x2064_M300_g32_act_4wave", "2048x4112_M400_4wave",
                               "4096x1040_M250_g64_32row", "4096x4112_M160_act_32row"])
 def test_prefill_128_row_tiles_partial(hip_device, k, n, m, g, act):
-    """The LDS-streamed kernel's tile shapes -- 64 x 256 (M = 300 at K = 1024),
-    128 x 128 (M = 520 .. 1000), 128 x 256 (M = 2000, where it needs fewer
-    rounds of workgroups), the 4-wave 64 x 128 workgroups that K <= 4096
-    takes where they need fewer K splits (M = 300, 400) and the 4-wave
-    32 x 128 workgroups of M <= 256 at K <= 4096 -- with a partial last row
-    tile, a partial last column tile (N not a multiple of the tile width) and
-    group sizes 32 / 64 / 128, unsplit and split along K (the splits of a
-    column tile spread over the XCDs as units of their own)."""
+    """The prefill path from 160 to 2000 rows with a partial last row tile, a
+    partial last column tile (N not a multiple of the tile width) and group
+    sizes 32 / 64 / 128, unsplit and split along K (the splits of a column
+    tile spread over the XCDs as units of their own).  The planner's tiles,
+    unsplit: K-sliced 64 x 32, 32 x 64 and 64 x 64 for the narrow and small
+    ones, LDS-streamed 64 x 128 (M = 400) and 96 x 256 (M = 1000, 2000); the
+    ids name the tiles of an earlier plan (test_gpu_prefill_tiles.py asserts
+    a case's tile)."""
     lay, w = oracle_w(k, n, g, 5000 + m, False, act)
     q4 = build(lay, hip_device)
     for split in (0, 1, 2):
@@ -408,14 +409,12 @@ def test_prefill_128_row_tiles_partial(hip_device, k, n, m, g, act):
                          ids=["32x128_M200", "32x128_M256", "64x256_K11008_M200",
                               "128x128_M600", "128x256_M2000"])
 def test_prefill_bias_lds_streamed_tiles(hip_device, k, n, m):
-    """Bias in the LDS-streamed kernel's epilogues, unsplit (split 1: the
-    tile's own epilogue adds it) and split along K (automatic and 2: the
+    """Bias in the prefill kernels' epilogues, unsplit (split 1: the tile's own
+    epilogue adds it) and split along K (2, and the plan's own choice: the
     reduce adds it), against the oracle plus bias.  The planner's tiles for
-    these shapes: the 4-wave 32 x 128 workgroups at K = 4096 and M <= 256
-    (a partial last column tile at N = 1040), the 8-wave 64 x 256 at
-    K = 11008 and M = 200 (K beyond 4096 keeps the 8-wave tiles), 128 x 128
-    at M = 600 (above 512 rows; one round of 45 tiles) and 128 x 256 at
-    M = 2000, N = 4112 (two rounds against three for 128 x 128)."""
+    these shapes: K-sliced 64 x 32 (K = 4096, M <= 256), 64 x 64 in three
+    splits (K = 11008) and unsplit (M = 600), LDS-streamed 96 x 256 (M = 2000);
+    the ids name the tiles of an earlier plan."""
     lay, w = oracle_w(k, n, 128, 6060 + m, False, False)
     q4 = build(lay, hip_device)
     bias = (torch.randn(n, generator=torch.Generator().manual_seed(6)) * 0.5).half()
@@ -697,7 +696,7 @@ def test_bf16_native_decode(hip_device, k, n, g, sym, act):
     added after the bf16 rounding, equal bits on a repeat; q4.matmul returns
     exactly what the C entry point writes; act-order without workspace room
     (every workgroup gathering) gives the same bits; one row past the limit
-    takes the dense route."""
+    takes the prefill kernels' bf16 form (dw4_gemm_bf16_prefill)."""
     lay, w = oracle_w(k, n, g, 7100 + k + n, sym, act)
     a = lay.numpy()
     wb = gptq.bf16_to_float(gptq.dequantize_bf16(a["qweight"], a["qzeros"], a["scales"],

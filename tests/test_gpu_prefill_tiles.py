@@ -82,6 +82,8 @@ CASES = [
     (600, 256, 8208, 128, False, "L 96x256/1"),
     (385, 512, 8208, 64, False, "L 64x256/1"),   # one row in the last tile
     (1300, 384, 4112, 32, False, "L 96x256/1"),
+    (500, 7552, 8192, 128, False, "L 128x128/1"),
+    (520, 13824, 2064, 64, True, "L 96x256/4"),
 ]
 
 

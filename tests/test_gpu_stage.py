@@ -112,9 +112,10 @@ def test_gemm_group_mixed_widths(hip_device):
 
 @pytest.mark.parametrize("case", ["qkv", "gate_up", "partial_tiles", "split_fallback"])
 def test_gemm_group_prefill(hip_device, case):
-    """Above 128 rows, matrices of equal N in one LDS-streamed prefill launch
-    (planned for the summed N), each with its own output and bias; the
-    plans that would split K run the matrices one after another."""
+    """Above the decode sizes, matrices of equal N in one launch of the
+    LDS-streamed or K-sliced kernel over all their column tiles, each with its
+    own output and bias, or one after another (each with its own K split)
+    where the plan's model prefers that."""
     import ctypes
 
     from hip_extends.w4a16 import _item

@@ -6,9 +6,10 @@ library's fixed per-GPU scratch array instead of a caller workspace, so its
 output must equal dw4_gemm's bit for bit.  Two calls in a row, the second
 smaller, check that what the first left in the shared array does not leak
 into the second; a call needing more than the array is refused before any
-launch.  The register-fed prefill kernel's in-kernel split-K (M of 33-128
-rows) keeps per-tile arrival counters at the head of the array, which every
-call must leave at zero: two such calls in a row check that.  A call
+launch.  The register-fed prefill kernel's in-kernel split-K (act-order up
+to 64 rows beyond the decode sizes) keeps per-tile arrival counters at the
+head of the array, which every call must leave at zero: two such calls in a
+row check that.  A call
 captured into a HIP graph (after one eager call has set the array up on the
 device) replays to the same bits.
 """
@@ -66,14 +67,16 @@ def _both(q4, m, seed):
 
 @pytest.mark.parametrize("act", [False, True], ids=["plain", "act"])
 def test_noalloc_matches_gemm_two_calls(hip_device, act):
-    """First call: M=256 on 8192x4096 (the LDS-streamed prefill kernel split
-    over K: fp32 partial planes in the scratch, summed by a second kernel;
-    act-order also gathers x there).  Second call, smaller: M=40 on
-    4096x2048, then M=1 decode."""
+    """M=256 on 8192x4096 (the K-sliced kernel; act-order gathers x into the
+    scratch), then smaller calls: M=40 on 4096x2048, M=1 decode; then M=700
+    (the LDS-streamed kernel split over K: fp32 partial planes in the scratch,
+    summed by a second kernel) and M=256 again."""
     big = _matrix(hip_device, 8192, 4096, act, 61)
     small = _matrix(hip_device, 4096, 2048, act, 62)
     assert _lib.workspace_size(256, 8192, 4096, 128, False) > 0  # the scratch is really used
-    for q4, m in ((big, 256), (small, 40), (small, 1), (big, 256)):
+    p = _lib.prefill_plan(700, 8192, 4096, 128, act, _lib.NOALLOC_SCRATCH_BYTES)
+    assert p.kernel == 1 and p.splits > 1
+    for q4, m in ((big, 256), (small, 40), (small, 1), (big, 700), (big, 256)):
         say(f"noalloc vs gemm {q4.height}x{q4.width} M={m} act={act}")
         y_ref, y = _both(q4, m, seed=m + 3 * act)
         assert not torch.isnan(y).any()
@@ -81,15 +84,23 @@ def test_noalloc_matches_gemm_two_calls(hip_device, act):
 
 
 def test_noalloc_split_counters_return_to_zero(hip_device):
-    """M=96 on 4096x4096 runs the register-fed prefill kernel split over K,
-    whose last-arriving split of each tile sums the partials and resets that
-    tile's arrival counter at the head of the scratch.  Two calls in a row
-    (then one with M=72) equal dw4_gemm bit for bit: a counter left non-zero
-    by the first call would make the second call's sums start early."""
+    """Act-order M=56 on 4096x8192 runs the register-fed prefill kernel split
+    over K, whose last-arriving split of each tile sums the partials and
+    resets that tile's arrival counter at the head of the scratch.  Two calls
+    in a row (then one with M=50) equal dw4_gemm bit for bit: a counter left
+    non-zero by the first call would make the second call's sums start early.
+    (Then M=96 and 72 without act-order: the K-sliced kernel.)"""
+    q4 = _matrix(hip_device, 4096, 8192, True, 63)
+    p = _lib.prefill_plan(56, 4096, 8192, 128, True, _lib.NOALLOC_SCRATCH_BYTES)
+    assert p.kernel == 0 and p.splits > 1  # counters in use
+    for m in (56, 56, 50):
+        say(f"noalloc vs gemm split counters 4096x8192 act M={m}")
+        y_ref, y = _both(q4, m, seed=m)
+        assert not torch.isnan(y).any()
+        assert torch.equal(y.view(torch.int16), y_ref.view(torch.int16)), f"M={m}"
     q4 = _matrix(hip_device, 4096, 4096, False, 63)
-    assert _lib.workspace_size(96, 4096, 4096, 128, False) > 0  # split: counters in use
     for m in (96, 96, 72):
-        say(f"noalloc vs gemm split counters 4096x4096 M={m}")
+        say(f"noalloc vs gemm 4096x4096 M={m}")
         y_ref, y = _both(q4, m, seed=m)
         assert not torch.isnan(y).any()
         assert torch.equal(y.view(torch.int16), y_ref.view(torch.int16)), f"M={m}"
