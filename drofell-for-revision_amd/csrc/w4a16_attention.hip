@@ -599,15 +599,15 @@ __global__ void reshape_and_cache_kernel(uint16_t* __restrict__ key, int64_t key
 //     16-byte aligned) as 2-byte elements.  Tiles start slots[0] % 8 tokens
 //     early, so a run that continues a half-filled cell still meets the
 //     tile in whole cells.
-// Measured, 1500 tokens x 32 heads x 128 written and read back: 67.7 -> 25.8 us
+// Measured, 1500 tokens x 32 heads x 128 written and read back: 67.7 -> 22.4 us
 // against element-wise copies (2-byte stores, one workgroup per token).
 constexpr int kCacheTile = 32;                 // tokens per workgroup
 constexpr int kCacheSlab = 128;                // dims per pass
 constexpr int kCachePitch = kCacheSlab + 4;    // halfs per LDS row: the 4 cells of a dim pair
                                                // read 4 x 16 distinct banks
 
-template <bool RESTORE>
-__global__ void __launch_bounds__(256)
+template <bool RESTORE, int THREADS>
+__global__ void __launch_bounds__(THREADS)
 cache_tile_kernel(uint16_t* __restrict__ key, int64_t key_stride, uint16_t* __restrict__ value,
                   int64_t value_stride, const int64_t* __restrict__ kptr,
                   const int64_t* __restrict__ vptr, const int64_t* __restrict__ slots,
@@ -652,7 +652,7 @@ cache_tile_kernel(uint16_t* __restrict__ key, int64_t key_stride, uint16_t* __re
     const int nd = min(kCacheSlab, head_size - d0);  // a multiple of 8
     const int nu = nd / 8;
     // ---- keys, 16-byte units: 8 tokens x 8 units per wave
-    for (int i = tid; i < kCacheTile * (kCacheSlab / 8); i += 256) {
+    for (int i = tid; i < kCacheTile * (kCacheSlab / 8); i += THREADS) {
       const int w = i >> 6, l = i & 63;
       const int t = (w & 3) * 8 + (l & 7);
       const int u = (w >> 2) * 8 + (l >> 3);
@@ -669,29 +669,26 @@ cache_tile_kernel(uint16_t* __restrict__ key, int64_t key_stride, uint16_t* __re
     }
     // ---- values
     auto rows = [&](auto&& move) {  // (tile address, row address) per 16-byte unit of a token
-      for (int i = tid; i < kCacheTile * (kCacheSlab / 8); i += 256) {
+      for (int i = tid; i < kCacheTile * (kCacheSlab / 8); i += THREADS) {
         const int t = i / (kCacheSlab / 8), u = i % (kCacheSlab / 8);
         if (u >= nu || vbase[t] == nullptr) continue;
         move(&tile[t * kCachePitch + u * 8], vrow + (size_t)(t0 + t) * value_stride + d0 + u * 8);
       }
     };
     auto cells = [&](auto&& move) {  // (tile address of the cell's first token, cache address)
-      for (int i = tid; i < (kCacheTile / 8) * (kCacheSlab / 2); i += 256) {
+      for (int i = tid; i < (kCacheTile / 8) * (kCacheSlab / 2); i += THREADS) {
         const int c = i % (kCacheTile / 8), dp = i / (kCacheTile / 8);
         if (2 * dp >= nd || !cell_ok[c]) continue;
         move(&tile[c * 8 * kCachePitch + 2 * dp],
              vbase[c * 8] + (size_t)(d0 + 2 * dp) * bs + (int)(slot_s[c * 8] & off_mask));
       }
     };
-    auto elements = [&](auto&& move) {  // tokens outside whole cells
-      if (!singles) return;
-      for (int i = tid; i < kCacheTile * kCacheSlab; i += 256) {
-        const int t = i % kCacheTile, d = i / kCacheTile;
-        if (d >= nd || cell_ok[t >> 3] || vbase[t] == nullptr) continue;
-        move(&tile[t * kCachePitch + d],
-             vbase[t] + (size_t)(d0 + d) * bs + (int)(slot_s[t] & off_mask));
-      }
-    };
+    // tokens outside whole cells: a thread's token, and its dims kStep apart
+    const int et = tid % kCacheTile;
+    const bool single = singles && !cell_ok[et >> 3] && vbase[et] != nullptr;
+    uint16_t* const erow = tile + et * kCachePitch;
+    uint16_t* const ecol = single ? vbase[et] + (size_t)d0 * bs + (int)(slot_s[et] & off_mask) : nullptr;
+    constexpr int kStep = THREADS / kCacheTile, kEach = kCacheSlab / kStep;
     if (!RESTORE) {
       rows([](uint16_t* lds, const uint16_t* row) {
         const u4 v = *(const u4*)row;
@@ -711,7 +708,8 @@ cache_tile_kernel(uint16_t* __restrict__ key, int64_t key_stride, uint16_t* __re
         *(u4*)dst = lo;
         *(u4*)(dst + bs) = hi;
       });
-      elements([](const uint16_t* lds, uint16_t* dst) { *dst = *lds; });
+      if (single)
+        for (int d = tid / kCacheTile; d < nd; d += kStep) ecol[(size_t)d * bs] = erow[d];
     } else {
       cells([&](uint16_t* lds, const uint16_t* src) {
         const u4 lo = *(const u4*)src, hi = *(const u4*)(src + bs);
@@ -721,7 +719,19 @@ cache_tile_kernel(uint16_t* __restrict__ key, int64_t key_stride, uint16_t* __re
           *(uint32_t*)(lds + (2 * e + 1) * kCachePitch) = (lo[e] >> 16) | (hi[e] & 0xFFFF0000u);
         }
       });
-      elements([](uint16_t* lds, const uint16_t* src) { *lds = *src; });
+      if (single) {  // all loads in flight before the first is stored
+        uint16_t v[kEach];
+#pragma unroll
+        for (int i = 0; i < kEach; ++i) {
+          const int d = tid / kCacheTile + i * kStep;
+          v[i] = d < nd ? ecol[(size_t)d * bs] : (uint16_t)0;
+        }
+#pragma unroll
+        for (int i = 0; i < kEach; ++i) {
+          const int d = tid / kCacheTile + i * kStep;
+          if (d < nd) erow[d] = v[i];
+        }
+      }
       __syncthreads();
       rows([](const uint16_t* lds, uint16_t* row) {
         const uint2 a = *(const uint2*)lds, b = *(const uint2*)(lds + 4);
@@ -997,16 +1007,29 @@ hipError_t launch_reshape_and_cache(uint16_t* key, int64_t key_stride, uint16_t*
                                     const int64_t* slots, int num_tokens, int num_kv_heads,
                                     int head_size, int block_size, int kv_head_stride,
                                     bool restore, hipStream_t stream) {
-  // whole 16-byte units on the rows' side (the kernel itself checks the
-  // blocks' addresses); rows that are not take the element-wise copy
+  // The tiles need whole 16-byte units on the rows' side (the kernel itself
+  // checks the blocks' addresses), and take 3 us for a single token; the
+  // element-wise copy, a workgroup of up to 1024 lanes per token, starts faster
+  // the narrower a row is.  Runs of tokens written and read back, element-wise
+  // against tiles (us): 8 heads of 128 256 tokens 7.6 / 8.0, 512 11.0 / 8.0; 16
+  // of 128 128 tokens 8.7 / 8.1, 256 11.1 / 8.2; 32 of 128 1 token 8.9 / 6.5, 64
+  // 12.4 / 8.0, 1500 67 / 22.  Tokens one to a block, which neither form can
+  // read or write in whole units, lose some us to the tile's steps in between:
+  // 32 of 128 64 tokens 14.0 / 15.9, 256 55 / 62, 1500 350 / 350.
   const bool vec = ((reinterpret_cast<uintptr_t>(key) | reinterpret_cast<uintptr_t>(value)) & 15) == 0 &&
                    key_stride % 8 == 0 && value_stride % 8 == 0;
-  if (vec) {
+  const bool wide = num_kv_heads * head_size / 8 + (int64_t)num_tokens >= 512;
+  if (vec && wide) {
     const dim3 grid((unsigned)((num_tokens + 7 + kCacheTile - 1) / kCacheTile), (unsigned)num_kv_heads);
     const int bs_log2 = block_size == 16 ? 4 : 5;
-    auto kern = restore ? &cache_tile_kernel<true> : &cache_tile_kernel<false>;
-    kern<<<grid, 256, 0, stream>>>(key, key_stride, value, value_stride, kptr, vptr, slots,
-                                   num_tokens, head_size, bs_log2, kv_head_stride);
+    // up to four workgroups per CU of 256 eight waves each, to have more copies
+    // in flight (512 tokens of 32 x 128 13.8 -> 11.9 us); beyond that four
+    // (1500 tokens 24.3 -> 22.4)
+    const bool few = (int64_t)grid.x * grid.y <= 1024;
+    auto kern = restore ? (few ? &cache_tile_kernel<true, 512> : &cache_tile_kernel<true, 256>)
+                        : (few ? &cache_tile_kernel<false, 512> : &cache_tile_kernel<false, 256>);
+    kern<<<grid, few ? 512 : 256, 0, stream>>>(key, key_stride, value, value_stride, kptr, vptr, slots,
+                                               num_tokens, head_size, bs_log2, kv_head_stride);
     return hipGetLastError();
   }
   const int n = num_kv_heads * head_size;

@@ -50,9 +50,12 @@ SLOTS = {
 
 @pytest.mark.parametrize("slots", SLOTS, ids=lambda s: s.replace(" ", "-"))
 @pytest.mark.parametrize("bs,kvh,hs,row_pad,block_pad", [
+    # narrow rows of few tokens, and rows 2-byte aligned: the element-wise kernel
     (16, 4, 128, 0, 0), (32, 3, 64, 8, 0), (32, 2, 256, 0, 0), (16, 2, 40, 0, 0),
-    (16, 2, 128, 3, 0),   # token rows 2-byte aligned: the element-wise kernel
-    (32, 2, 128, 0, 1),   # blocks 2-byte aligned: no 16-byte units on the cache side
+    (16, 2, 128, 3, 0), (32, 2, 128, 0, 1), (16, 32, 128, 3, 0),
+    # the tiles
+    (16, 32, 128, 0, 0), (32, 64, 64, 8, 0), (32, 16, 256, 0, 0), (16, 104, 40, 0, 0),
+    (32, 32, 128, 0, 1),  # blocks 2-byte aligned: no 16-byte units on the cache side
 ])
 def test_cache_tile_edges(hip_device, slots, bs, kvh, hs, row_pad, block_pad):
     say(f"cache tile {slots} bs={bs} heads={kvh} hs={hs} pads={row_pad},{block_pad}")
@@ -109,3 +112,29 @@ def test_dequant_tile_edges(hip_device, k, n, g, act, pad, bf16):
     got = w.cpu().numpy().view(np.uint16)
     assert np.array_equal(got[:, :n], ref)
     assert (got[:, n:] == 0xFFFF).all()  # the padding between rows is not written
+
+
+@pytest.mark.parametrize("n,kvh,hs,bs", [(383, 8, 128, 16), (384, 8, 128, 16), (448, 8, 64, 32), (500, 2, 80, 32),
+                                         (1013, 32, 64, 16), (1050, 32, 64, 16)])
+def test_cache_rules(hip_device, n, kvh, hs, bs):
+    """Both sides of the lines between the element-wise copy and the tiles
+    (narrow rows of few tokens) and between their 512 and 256 threads (up to
+    1024 workgroups), in runs that begin inside a cell."""
+    say(f"cache {n} x {kvh} x {hs} bs={bs}")
+    sl = _runs(bs, 3, [n // 3, n // 2, n - n // 3 - n // 2])
+    blocks, per = int(sl.max()) // bs + 1, kvh * hs * bs
+    rng = np.random.default_rng(n)
+    key, val = (rng.standard_normal((n, kvh, hs)).astype(np.float16) for _ in range(2))
+    kc, vc = A.empty_cache(blocks, kvh, hs, bs, fill=0.0)
+    A.reshape_and_cache(key, val, kc, vc, sl)
+    bufs = [torch.zeros(blocks * per, dtype=torch.float16, device=hip_device) for _ in range(2)]
+    ptrs = [torch.arange(blocks, dtype=torch.int64, device=hip_device) * (2 * per) + b.data_ptr() for b in bufs]
+    rows = [torch.from_numpy(a.reshape(n, -1)).to(hip_device) for a in (key, val)]
+    back = [torch.zeros_like(r) for r in rows]
+    sd, stream = torch.from_numpy(sl).to(hip_device), torch.cuda.current_stream().cuda_stream
+    for name, r in (("dw4_reshape_and_cache", rows), ("dw4_restore_from_cache", back)):
+        _lib.call(name, n, kvh, hs, bs, r[0].data_ptr(), r[0].stride(0), r[1].data_ptr(), r[1].stride(0),
+                  ptrs[0].data_ptr(), ptrs[1].data_ptr(), hs * bs, sd.data_ptr(), stream)
+    for buf, ref in zip(bufs, (kc, vc)):
+        assert np.array_equal(buf.cpu().numpy().view(np.uint16), ref.reshape(-1).view(np.uint16))
+    assert all(torch.equal(a, b) for a, b in zip(rows, back))
