@@ -558,12 +558,17 @@ GemmTPlan plan_gemm_t(int m, int k, int n, int cus) {
 // The route this replaces writes and reads the dense weight (8 us + 1.07 us
 // per million weights, at least 20 for its two launches) and runs a library
 // product (1.35e-3 us per row and million weights).  Groups under 128 rows cost
-// the tall form a fifth more.  Measured, packed against dense: 4096 x 11008
-// M = 192 36 / 88, 256 46 / 67, 384 58 / 76, 512 73 / 86, 768 112 / 102; 4096^2
-// M = 384 26 / 37, 512 33 / 40, 768 49 / 44; 11008 x 4096 in groups of 64
-// M = 192 57 / 61, 256 67 / 69, 384 86 / 69; 5120 x 13824 M = 384 93 / 113,
-// 512 138 / 130.  With buffers out of cache, in training, 384 rows on 4096 x 11008
-// take 66 us packed and the dense route 68, so the line lies at 0.6 of its time.
+// the tall form a fifth more.  Measured (us, packed / dense with the weight
+// just written / dense over weights out of cache, matrices and rows rotated in
+// both): 4096 x 11008 M = 192 37 / 89 / 126, 256 45 / 67 / 86, 384 57 / 76 / 96, 512
+// 73 / 87 / 110; 4096^2 M = 192 20 / 40 / 47, 384 26 / 34 / 39, 512 32 / 38 / 43; 11008 x
+// 4096 M = 192 47 / 60 / 75, 320 61 / 67 / 83, 384 73 / 68 / 83; in groups of 64 M =
+// 160 58 / 56 / 72, 320 68 / 66 / 84; 5120 x 13824 M = 256 77 / 145 / 193, 384 103 / 115 /
+// 143, 512 142 / 143 / 164.  The line at 0.6 of the modelled dense time is a
+// cautious one: it takes the packed words only where they are ahead by more
+// than the model's error on every shape (up to 192 rows on 4096 x 11008, 128 on
+// 4096^2), and leaves a band above it, to about 384 rows, where they are
+// ahead by 1.1 to 2.
 bool gemm_t_beats_dense(const GemmTPlan& p, int m, int k, int n, int gs) {
   if (p.mt == 0) return true;
   const double mw = 1e-6 * k * n;
