@@ -1022,10 +1022,10 @@ hipError_t launch_reshape_and_cache(uint16_t* key, int64_t key_stride, uint16_t*
   if (vec && wide) {
     const dim3 grid((unsigned)((num_tokens + 7 + kCacheTile - 1) / kCacheTile), (unsigned)num_kv_heads);
     const int bs_log2 = block_size == 16 ? 4 : 5;
-    // up to four workgroups per CU of 256 eight waves each, to have more copies
-    // in flight (512 tokens of 32 x 128 13.8 -> 11.9 us); beyond that four
-    // (1500 tokens 24.3 -> 22.4)
-    const bool few = (int64_t)grid.x * grid.y <= 1024;
+    // up to three workgroups per CU (of 256) eight waves each, to have more
+    // copies in flight (32 x 128, us, four / eight waves: 512 tokens 13.8 / 11.9,
+    // 700 15.1 / 13.5); beyond that four (800 tokens 15.3 / 17.3, 1500 22.1 / 24.3)
+    const bool few = (int64_t)grid.x * grid.y <= 768;
     auto kern = restore ? (few ? &cache_tile_kernel<true, 512> : &cache_tile_kernel<true, 256>)
                         : (few ? &cache_tile_kernel<false, 512> : &cache_tile_kernel<false, 256>);
     kern<<<grid, few ? 512 : 256, 0, stream>>>(key, key_stride, value, value_stride, kptr, vptr, slots,

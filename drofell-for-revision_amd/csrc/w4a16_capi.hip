@@ -163,8 +163,12 @@ dw4::PrefillPlan plan_prefill(int m, int k, int n, int split_req, size_t ws_byte
 // of the last round run faster the fewer CUs it fills (clocks, L2).  A K split
 // adds the reduce launch and its fp32 planes (us per MB).  The constants (us)
 // are least-squares fits to 3024 graph-replayed launches: seven 7B and 13B
-// shapes, M = 24..3500, splits 1..8, 256 CUs; mean error 2-4 % per tile, and
-// on the 126 (shape, M > 64) points the pick is 0.1 % slower than the fastest
+// shapes, M = 24..3500, splits 1..8, 256 CUs.  Measured again (5128 launches,
+// 98 points of seven shapes and M = 40..3500; profiles/prefill_tiles.csv holds
+// those within half again of their point's best): the model is off by 2-4 % per
+// tile in the mean where a tile is within a quarter of the best, by more where
+// it is far from it (K-sliced tiles above a few hundred rows, 5 % too slow on
+// 64 x 128), and the pick is 0.3 % slower in the geometric mean than the fastest
 // launch measured.  Against the rules this replaces (fewest rounds, fixed
 // preferences by M) the picks are 1.13x faster in the geometric mean:
 // 4096^2 M=256 21.1 -> 16.4 us, 5120^2 M=96 19.9 -> 13.2, 4096 x 11008 M=384

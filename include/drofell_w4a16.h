@@ -195,8 +195,8 @@ int dw4_gemm(int m, int k, int n, int group_size,
 
 /* Device: y[M, N] = bf16(x[M, K] @ W) (+ bias[N] in bf16, added after that
  * rounding) for bf16 activations x and a bf16 output y, 1 <= m <=
- * DW4_BF16_MAX_M; larger m returns DW4_ERR_UNSUPPORTED (the caller keeps
- * the dense route: dw4_dequant_bf16, then a bf16 library GEMM).  One
+ * DW4_BF16_MAX_M; larger m returns DW4_ERR_UNSUPPORTED (the caller takes
+ * dw4_gemm_bf16_prefill, or dw4_dequant_bf16 and a bf16 library GEMM).  One
  * register-fed decode launch on bf16 matrix cores (every row tile of 16 rows
  * in the same launch, the packed weights read once), fp32 accumulation over
  * the exact integers q - z and the fp16 scales applied per group in fp32, so

@@ -115,11 +115,11 @@ def test_dequant_tile_edges(hip_device, k, n, g, act, pad, bf16):
 
 
 @pytest.mark.parametrize("n,kvh,hs,bs", [(383, 8, 128, 16), (384, 8, 128, 16), (448, 8, 64, 32), (500, 2, 80, 32),
-                                         (1013, 32, 64, 16), (1050, 32, 64, 16)])
+                                         (761, 32, 64, 16), (762, 32, 64, 16)])
 def test_cache_rules(hip_device, n, kvh, hs, bs):
     """Both sides of the lines between the element-wise copy and the tiles
     (narrow rows of few tokens) and between their 512 and 256 threads (up to
-    1024 workgroups), in runs that begin inside a cell."""
+    768 workgroups), in runs that begin inside a cell."""
     say(f"cache {n} x {kvh} x {hs} bs={bs}")
     sl = _runs(bs, 3, [n // 3, n // 2, n - n // 3 - n // 2])
     blocks, per = int(sl.max()) // bs + 1, kvh * hs * bs
