@@ -7,6 +7,7 @@ object is missing or fails to load, every entry point raises.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 import threading
 from typing import Optional
@@ -157,6 +158,8 @@ class W4A16Error(RuntimeError):
 def load(path: str = LIB_PATH) -> ctypes.CDLL:
     """Load (once) and type the native library; raises if it is absent."""
     global _lib
+    if _lib is not None:
+        return _lib
     with _lock:
         if _lib is not None:
             return _lib
@@ -252,7 +255,11 @@ def gemm_t_packed(m: int, k: int, n: int, group_size: int) -> bool:
     return out.value != 0
 
 
-def gemm_t_workspace_size(m: int, k: int, n: int, group_size: int) -> int:
+@functools.lru_cache(maxsize=4096)
+def gemm_t_workspace_size(m: int, k: int, n: int, group_size: int,
+                          device: Optional[int] = None) -> int:
+    """Bytes of dw4_gemm_t's planes on the current device (``device``, its
+    index, only tells the remembered sizes of several devices apart)."""
     lib = load()
     out = ctypes.c_size_t(0)
     check("dw4_gemm_t_workspace_size",

@@ -30,7 +30,7 @@ from dataclasses import dataclass
 from typing import Any, Dict, Optional, Tuple
 
 import torch
-from torch.autograd import Function
+from torch.autograd import Function, forward_ad
 
 from . import _lib
 
@@ -134,7 +134,7 @@ def _untracked(t: torch.Tensor) -> bool:
     for it, no vmap or other transform wraps it and it carries no tangent."""
     return not (t.requires_grad and torch.is_grad_enabled()) \
         and not torch._C._functorch.is_functorch_wrapped_tensor(t) \
-        and torch.autograd.forward_ad.unpack_dual(t).tangent is None
+        and (forward_ad._current_level < 0 or forward_ad.unpack_dual(t).tangent is None)
 
 
 def _aligned_rows(x2: torch.Tensor) -> torch.Tensor:
@@ -448,12 +448,13 @@ class Q4MatrixV2(object):
         m = g2.shape[0]
         out2 = torch.empty((m, self.height), dtype=torch.float16, device=device) \
             if output is None else _output_rows(output, m, self.height, torch.float16)
-        nbytes = _lib.gemm_t_workspace_size(m, self.height, self.width, self.group_size)
-        ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=device)
+        nbytes = _lib.gemm_t_workspace_size(m, self.height, self.width, self.group_size,
+                                            device.index)
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=device) if nbytes else None
         _lib.call("dw4_gemm_t", m, self.height, self.width, self.group_size,
                   g2.data_ptr(), g2.stride(0), qweight.data_ptr(), qzeros.data_ptr(),
                   scales.data_ptr(), _ptr(perm) if self.use_act else None,
-                  out2.data_ptr(), out2.stride(0), ws.data_ptr(), ws.numel(), _stream(device))
+                  out2.data_ptr(), out2.stride(0), _ptr(ws), nbytes, _stream(device))
         return out2.view(outshape) if output is None else output
 
     def _dense_weight(self, temp_weight: Optional[torch.Tensor],
@@ -592,7 +593,7 @@ class Q4LinearFunction(Function):
     the backward (unless the matrix already holds a reconstructed one).  Where
     the backward runs on the packed words (fp16 rows up to the library's rule,
     where writing the dense weight costs more than it saves: 128 rows on
-    4096 x 11008 74 us to write and use, against 29 packed), the packed
+    4096 x 11008 96 us to write and use, against 31 packed), the packed
     tensors are saved in its place, so the gradient is that of the forward's
     weight whatever the matrix has been pointed at since, and autograd
     refuses it if they were overwritten.
